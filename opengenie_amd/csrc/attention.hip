@@ -84,7 +84,7 @@ struct AttnArgs {
   int64_t nq, nk;
   int heads;
   int nqb;        // query blocks per (batch, head)
-  int qpb;        // queries per block (kAQ, or kF8Q for the FP8 kernel)
+  int qpb;        // queries per block (32 per wave of the kernel's workgroup)
   int xcd_remap;  // nfull divisible by the 8 XCDs
   float scale_log2;  // softmax scale * log2(e)
   // Workgroups 0 .. nfull-1 each own query block blockIdx.x (remapped) over
@@ -855,9 +855,13 @@ __global__ __launch_bounds__(64 * kFewW) __attribute__((amdgpu_waves_per_eu(2, 2
 constexpr int kF8Tile = kAK * kAD;  // bytes of a K or V^T tile: 8 KiB
 constexpr float kF8Offset = 8.0f;  // P = 2^(s - m + kF8Offset): a row's largest P is >= 256
 // How far a row's scores may pass the running max before O and l are
-// rescaled: 2^(8 + 0.8) = 445.7 stays below e4m3's largest finite 448.
-constexpr float kF8Lag = 0.8f;
-static_assert(kF8Offset + kF8Lag < 8.807f, "P must stay below 448 = 2^8.807");
+// rescaled: at most 0.8, as 2^(8 + 0.8) = 445.7 stays below e4m3's largest
+// finite 448. The narrow form below lags by nothing: every score that sets a
+// new maximum then has P = 256, exact in e4m3, and the error against float64
+// attention falls from 0.0256 to 0.0250 at 4999 tokens (0.0251 -> 0.0246 at
+// 2304) for 3 % more time (324 against 334 us for the whole call).
+constexpr float kF8WideLag = 0.8f;
+static_assert(kF8Offset + kF8WideLag < 8.807f, "P must stay below 448 = 2^8.807");
 constexpr int kF8Pair = 2 * kF8Tile;
 constexpr int k8_off(int r, int c) { return (r >> 1) * 256 + (((r & 1) * 8 + c) ^ ((r >> 1) & 7)) * 16; }
 constexpr int vt_off(int d, int c) { return d * 64 + ((c ^ ((d >> 2) & 3)) << 4); }
@@ -908,25 +912,40 @@ OGA_DEVICE i32x8 lds_b256(uint32_t a0, uint32_t a1) {
   return r;
 }
 
-#ifndef OGA_F8_WAVES
-#define OGA_F8_WAVES 12
-#endif
-constexpr int kF8W = OGA_F8_WAVES;  // waves per FP8 workgroup, 32 queries each
-constexpr int kF8Q = 32 * kF8W;      // queries per FP8 workgroup
-constexpr int kF8DmaW = 8;           // waves whose DMA fills the tiles: one 1 KiB instruction per tile each
-static_assert(kF8W == 8 || kF8W == 12, "8 waves (2 per SIMD) or 12 (3 per SIMD)");
-constexpr int kF8Bufs = kABufs;  // K/V^T tile pairs in the FP8 kernel's ring
-// Waves past the eighth send the same two DMA instructions per step as the
-// others (so that every wave waits for the same count) into 2 KiB of their
-// own after the ring, re-reading tile rows the first eight fetch.
-constexpr int kF8DummyOff = kF8Bufs * kF8Pair;
-constexpr int kF8Ring = kF8DummyOff + (kF8W - kF8DmaW) * 2048;
-constexpr int kF8Lds = kF8Ring > kF8W * 8192 ? kF8Ring : kF8W * 8192;
-static_assert(kF8Ring <= 65536, "the FP8 fragment reads address LDS with 16-bit offsets");
+// Two forms, three waves per SIMD in both: one workgroup of 12 waves (384
+// queries) per CU, or three of 4 waves (128 queries). The narrow one wastes
+// less of a last round and of a ragged last block, and needs no key split
+// where the wide one does (32 heads: 4999 tokens, 448 wide blocks = 1.75
+// rounds in key parts and a merge, 307 + 26 us; 1280 narrow ones 245 us). The
+// wide one fetches each K/V^T tile once per 384 queries, worth ~4 % where both
+// fill their rounds (9216 tokens: 866 against 900 us for the whole call).
+// fp8_kernel() takes the one whose modelled time is shorter.
+constexpr int kF8Wide = 12, kF8Narrow = 4;
+constexpr int kF8Bufs = 3;  // K/V^T tile pairs in the FP8 kernel's ring
+template <int W>
+struct F8Cfg {
+  static_assert(W == kF8Wide || W == kF8Narrow, "4 or 12 waves");
+  static constexpr int kQ = 32 * W;         // queries per workgroup
+  static constexpr int kPerCu = 12 / W;     // workgroups per CU
+  static constexpr float kLag = W == kF8Wide ? kF8WideLag : 0.0f;
+  static constexpr int kDmaW = W < 8 ? W : 8;  // waves whose DMA fills the tiles
+  static constexpr int kDI = 8 / kDmaW;     // 1 KiB instructions per wave and tile
+  // Waves past the eighth send the same DMA instructions per step as the
+  // others (so that every wave waits for the same count) into 2 KiB of their
+  // own after the ring, re-reading tile rows the first eight fetch.
+  static constexpr int kDummyOff = kF8Bufs * kF8Pair;
+  static constexpr int kRing = kDummyOff + (W - kDmaW) * 2048;
+  static constexpr int kLds = kRing > W * 8192 ? kRing : W * 8192;
+  static_assert(kRing <= 65536, "the FP8 fragment reads address LDS with 16-bit offsets");
+  static_assert(kPerCu * kLds <= 160 * 1024, "LDS budget of the workgroups of a CU");
+};
 
-__global__ __launch_bounds__(64 * kF8W) __attribute__((amdgpu_waves_per_eu(kF8W / 4, kF8W / 4))) void k_attention_fp8(
-    AttnArgs a) {
-  __shared__ uint4 smem[kF8Lds / 16];
+template <int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_attention_fp8(AttnArgs a) {
+  using Cfg = F8Cfg<W>;
+  constexpr int kF8Q = Cfg::kQ, kDmaW = Cfg::kDmaW, kDI = Cfg::kDI;
+  constexpr float kF8Lag = Cfg::kLag;
+  __shared__ uint4 smem[Cfg::kLds / 16];
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   int64_t wg = blockIdx.x;
@@ -973,11 +992,12 @@ __global__ __launch_bounds__(64 * kF8W) __attribute__((amdgpu_waves_per_eu(kF8W 
     for (int e = 0; e < 16; ++e) o[i][e] = 0.0f;
   float m_run = -INFINITY, l_run = 0.0f;
 
-  // DMA: wave wv fills bytes [1024 wv, 1024 wv + 1024) of each tile. K: lane
-  // p writes line L = 4wv + p/16, position p%16, holding row 2L + v/8, chunk
-  // v%8 with v = (p%16) ^ (L%8). V^T: lane p writes d-row 16wv + p/4,
-  // position p%4, holding chunk (p%4) ^ ((d/4)%4) of the row.
-  const int wd = wv % kF8DmaW;  // the tile part this wave's DMA reads
+  // DMA: instruction i (< kDI) of wave wd fills KiB p = wd + 4i of each tile.
+  // K: lane l writes line L = 4p + l/16, position l%16, holding row 2L + v/8,
+  // chunk v%8 with v = (l%16) ^ (L%8). V^T: lane l writes d-row 16p + l/4,
+  // position l%4, holding chunk (l%4) ^ ((d/4)%4) of the row. Instruction 1
+  // covers the K rows 32 and the d-rows 64 further, same chunks.
+  const int wd = wv % kDmaW;  // the tile part this wave's DMA reads
   const int kL = 4 * wd + (lane >> 4);
   const int kv = (lane & 15) ^ (kL & 7);
   const int krow = 2 * kL + (kv >> 3);
@@ -988,23 +1008,32 @@ __global__ __launch_bounds__(64 * kF8W) __attribute__((amdgpu_waves_per_eu(kF8W 
   // wave-uniform base, so a step's DMA addresses cost no 64-bit vector math.
   const uint32_t vt_src = (uint32_t)(vd_row * a.vt_npad) + (uint32_t)(((lane & 3) ^ ((vd_row >> 2) & 3)) * 16);
   const uint32_t k_src = (uint32_t)(krow * a.k_sn) + koff_c;
-  // LDS destinations (wave-uniform): the wave's 1 KiB of the pair's K and
-  // V^T tiles, or, for a wave past the eighth, its own 2 KiB after the ring.
-  const bool tile_wave = wv < kF8DmaW;
-  const int k_dst = tile_wave ? wv * 64 : kF8DummyOff / 16 + (wv - kF8DmaW) * 128;
-  const int v_dst = tile_wave ? kF8Tile / 16 + wv * 64 : kF8DummyOff / 16 + (wv - kF8DmaW) * 128 + 64;
+  const uint32_t k_sn32 = (uint32_t)(32 * a.k_sn), vt_64 = (uint32_t)(64 * a.vt_npad);
+  // LDS destinations (wave-uniform): the wave's KiB of the pair's K and V^T
+  // tiles, or, for a wave past the eighth, its own 2 KiB after the ring.
+  const bool tile_wave = wv < kDmaW;
+  const int k_dst = tile_wave ? wv * 64 : Cfg::kDummyOff / 16 + (wv - kDmaW) * 128;
+  const int v_dst = tile_wave ? kF8Tile / 16 + wv * 64 : Cfg::kDummyOff / 16 + (wv - kDmaW) * 128 + 64;
   auto dma_step = [&](int64_t s2, uint4* dst) {
     const int64_t key0 = s2 * kAK;
     uint4* const kd = tile_wave ? dst + k_dst : smem + k_dst;
     uint4* const vdp = tile_wave ? dst + v_dst : smem + v_dst;
+    const uint8_t* const kt = kbase + key0 * a.k_sn;
+    const uint8_t* const vtt = vtbase + key0;
     // Rows past the last key (the last, partial step) re-read the last key.
     const int last = (int)min((int64_t)(kAK - 1), a.nk - 1 - key0);
-    const uint32_t ko = krow <= last ? k_src : (uint32_t)(last * a.k_sn) + koff_c;
-    __builtin_amdgcn_global_load_lds((const void*)(kbase + key0 * a.k_sn + ko), (lds_void*)kd, 16, 0, 0);
-    __builtin_amdgcn_global_load_lds((const void*)(vtbase + key0 + vt_src), (lds_void*)vdp, 16, 0, 0);
+    const uint32_t kend = (uint32_t)(last * a.k_sn) + koff_c;
+#pragma unroll
+    for (int i = 0; i < kDI; ++i) {
+      const uint32_t ko = krow + 32 * i <= last ? k_src + i * k_sn32 : kend;
+      __builtin_amdgcn_global_load_lds((const void*)(kt + ko), (lds_void*)(kd + 256 * i), 16, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < kDI; ++i)
+      __builtin_amdgcn_global_load_lds((const void*)(vtt + (vt_src + i * vt_64)), (lds_void*)(vdp + 256 * i), 16, 0, 0);
   };
   dma_step(st_begin, smem);
-  if (kF8Bufs == 3) dma_step(min(st_begin + 1, st_end - 1), smem + kF8Pair / 16);
+  dma_step(min(st_begin + 1, st_end - 1), smem + kF8Pair / 16);
 
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void*)smem;
   uint32_t kaddr[2][2], vaddr[2];
@@ -1110,41 +1139,27 @@ __global__ __launch_bounds__(64 * kF8W) __attribute__((amdgpu_waves_per_eu(kF8W 
 
   auto step = [&](auto par_c, int64_t st) {
     constexpr int PAR = decltype(par_c)::value;
-    // This wave's two DMA instructions of step st have landed (those of
-    // step st + 1 may still be in flight), then every wave's.
-    if (kF8Bufs == 3)
-      asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // This wave's DMA of step st has landed (the last two instructions of
+    // step st + 1's, sent a step ago, may still be in flight), then every
+    // wave's.
+    asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
     asm volatile("s_barrier" ::: "memory");
-    {
-      constexpr int NP = (PAR + kF8Bufs - 1) % kF8Bufs;
-      if (kF8Bufs == 3)
-        dma_step(min(st + 2, st_end - 1), smem + NP * (kF8Pair / 16));
-      else if (st + 1 < st_end)
-        dma_step(st + 1, smem + NP * (kF8Pair / 16));
-    }
+    constexpr int NP = (PAR + kF8Bufs - 1) % kF8Bufs;
+    dma_step(min(st + 2, st_end - 1), smem + NP * (kF8Pair / 16));
     f32x16 sacc[2];
     i32x8 vf[4], pf;
     s_phase(par_c, sacc);
-    if constexpr (kF8W == 8) {
-      // V^T fragments in flight under the softmax.
-      v_read(par_c, vf);
-      softmax(st, sacc, pf);
-    } else {
-      // With three waves per SIMD the fragments are read after the softmax
-      // (168 VGPRs), the other waves covering the reads' latency.
-      softmax(st, sacc, pf);
-      v_read(par_c, vf);
-    }
+    // With three waves per SIMD the fragments are read after the softmax
+    // (168 VGPRs), the other waves covering the reads' latency.
+    softmax(st, sacc, pf);
+    v_read(par_c, vf);
     pv(vf, pf);
   };
 
   for (int64_t st = st_begin; st < st_end; st += kF8Bufs) {
     step(IC<0>{}, st);
     if (st + 1 < st_end) step(IC<1>{}, st + 1);
-    if constexpr (kF8Bufs == 3)
-      if (st + 2 < st_end) step(IC<2 % kF8Bufs>{}, st + 2);
+    if (st + 2 < st_end) step(IC<2>{}, st + 2);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
@@ -1318,8 +1333,8 @@ extern "C" int oga_fp8_dequant_per_head(const void* x8, const float* descale, vo
 
 namespace {
 // The attention kernels: the bf16 kernel for many keys and for few
-// (kShortSteps), and the FP8 kernel.
-enum AttnKernel { kBf16Long = 0, kBf16Short = 1, kFp8 = 2 };
+// (kShortSteps), and the two forms of the FP8 kernel.
+enum AttnKernel { kBf16Long = 0, kBf16Short = 1, kFp8Wide = 2, kFp8Narrow = 3 };
 struct AttnCfg {
   const void* fn;
   int threads, qpb;
@@ -1327,7 +1342,8 @@ struct AttnCfg {
 AttnCfg attn_cfg(AttnKernel k) {
   switch (k) {
     case kBf16Short: return {(const void*)k_attention<kAWShort, kABufsShort>, 64 * kAWShort, 32 * kAWShort};
-    case kFp8: return {(const void*)k_attention_fp8, 64 * kF8W, kF8Q};
+    case kFp8Wide: return {(const void*)k_attention_fp8<kF8Wide>, 64 * kF8Wide, F8Cfg<kF8Wide>::kQ};
+    case kFp8Narrow: return {(const void*)k_attention_fp8<kF8Narrow>, 64 * kF8Narrow, F8Cfg<kF8Narrow>::kQ};
     default: return {(const void*)k_attention<kAW, kABufs>, 64 * kAW, kAQ};
   }
 }
@@ -1337,7 +1353,7 @@ AttnKernel bf16_kernel(int64_t nk) { return (nk + kAK - 1) / kAK <= kShortSteps 
 // (CUs x workgroups per CU), cached per device (relaxed atomics: threads
 // filling an entry at once store the same value); 0 if the runtime cannot say.
 int64_t attention_slots(AttnKernel kern) {
-  static std::atomic<int64_t> cache[3][64];
+  static std::atomic<int64_t> cache[4][64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
   int64_t n = cache[kern][dev].load(std::memory_order_relaxed);
@@ -1356,27 +1372,86 @@ int64_t attention_slots(AttnKernel kern) {
 struct AttnPlan {
   int64_t wgs, nfull, units;  // query blocks, whole ones, split parts
   int ksplit;
+  double us;  // modelled time
 };
-// Blocks beyond the last whole round of the CUs are cut into k parts over
-// their key steps (k <= 8 and <= the steps) when that shortens the last
-// round by at least a tenth of a round: rem blocks in k parts take
-// ceil(k rem / slots) rounds of 1/k of a block's time. Not for kShortSteps
-// steps or fewer: a block's time is then mostly its Q loads and O stores,
-// which every part repeats, and the merge adds a launch (at 256 keys the
-// split ran 75.7 against 66.9 us unsplit).
-AttnPlan attention_plan(int64_t wgs, int64_t nk, int64_t slots) {
-  AttnPlan p{wgs, wgs, 0, 1};
-  const int64_t rem = slots > 0 ? wgs % slots : 0;
-  if (rem == 0) return p;
+// Blocks beyond the last whole round of the resident workgroups may be cut
+// into k parts over their key steps (k <= 8 and <= the steps). Not for
+// kShortSteps steps or fewer: a block's time is then mostly its Q loads and O
+// stores, which every part repeats, and the merge adds a launch (at 256 keys
+// the split ran 75.7 against 66.9 us unsplit). split_candidate is the k with
+// the shortest last round alone (ceil(k rem / slots) rounds of 1/k of a
+// block's time, shorter by at least a tenth of a round); it sizes the
+// workspace.
+int split_candidate(int64_t rem, int64_t nk, int64_t slots) {
   const int64_t nsteps = (nk + kAK - 1) / kAK;
-  if (nsteps <= kShortSteps) return p;
+  int ksplit = 1;
+  if (nsteps <= kShortSteps) return 1;
   double best = 1.0;
   for (int k = 2; k <= 8 && k <= nsteps; ++k) {
     const double c = (double)((k * rem + slots - 1) / slots) / k;
-    if (c < best - 0.1) { best = c; p.ksplit = k; }
+    if (c < best - 0.1) { best = c; ksplit = k; }
   }
+  return ksplit;
+}
+// Time of `units` units of `steps` key steps each, in us: rounds of the
+// resident workgroups, the last one at the step time of as many workgroups
+// per CU as it still needs. A step of one 8-wave bf16 workgroup takes ~1.6 us,
+// of one 12-wave FP8 workgroup ~1.65; of one, two or three 4-wave FP8
+// workgroups on a CU ~0.75, 1.2 and 1.72 us; a unit's Q loads, first tiles
+// and O stores ~4 us.
+double units_us(AttnKernel kern, int64_t units, double steps, int64_t slots) {
+  static constexpr double kNarrowStep[3] = {0.75, 1.2, 1.72};
+  const double full = kern == kFp8Narrow ? kNarrowStep[2] : kern == kFp8Wide ? 1.65 : 1.6;
+  double t = (double)(units / slots) * (steps * full + 4.0);
+  const int64_t rest = units % slots;
+  if (rest) {
+    const int per_cu = kern == kFp8Narrow ? (int)((rest * 3 + slots - 1) / slots) : 3;
+    t += steps * (per_cu < 3 ? kNarrowStep[per_cu - 1] : full) + 4.0;
+  }
+  return t;
+}
+// The split that is run: the candidate, or any smaller k, when the last
+// round and the merge together are shorter than the whole blocks. A part's
+// float32 partials (qpb x 130 x 4 bytes, written and read back at ~4.5 TB/s)
+// and the merge's launch (~3 us) are what a split costs: 224 blocks of 25
+// steps in 8 parts (1537 tokens, 32 heads; 1792 partials, 238 MB) ran 127 us
+// and 38 us of merge, where the rounds alone promised an eighth less.
+AttnPlan attention_plan(AttnKernel kern, int64_t wgs, int64_t nk, int64_t slots) {
+  AttnPlan p{wgs, wgs, 0, 1, 0.0};
+  if (slots <= 0) return p;
+  const int64_t rem = wgs % slots;
+  const double nsteps = (double)((nk + kAK - 1) / kAK);
+  p.us = units_us(kern, wgs, nsteps, slots);
+  if (rem == 0) return p;
+  const int kmax = split_candidate(rem, nk, slots);
+  const double whole = units_us(kern, wgs - rem, nsteps, slots);
+  double best = p.us - whole;
+  for (int k = 2; k <= kmax; ++k) {
+    const double merge = 3.0 + (double)(k * rem) * attn_cfg(kern).qpb * (kAD + 2) * 8 / 4.5e6;
+    const double c = units_us(kern, k * rem, nsteps / k, slots) + merge;
+    if (c < best) { best = c; p.ksplit = k; }
+  }
+  p.us = whole + best;
   if (p.ksplit > 1) { p.nfull = wgs - rem; p.units = rem * p.ksplit; }
   return p;
+}
+// The form of the FP8 kernel whose plan is the shorter one.
+AttnKernel fp8_kernel(int64_t batch, int64_t nq, int64_t nk, int64_t heads, AttnPlan* plan) {
+  AttnKernel best = kFp8Wide;
+  for (AttnKernel kern : {kFp8Wide, kFp8Narrow}) {
+    const int qpb = attn_cfg(kern).qpb;
+    const AttnPlan p = attention_plan(kern, (nq + qpb - 1) / qpb * heads * batch, nk, attention_slots(kern));
+    if (kern == kFp8Wide || p.us < plan->us) { *plan = p; best = kern; }
+  }
+  return best;
+}
+// Bytes of partials the largest split of this shape could take: an upper
+// bound of what attention_plan uses, which keeps blocks whole where the
+// merge would cost more than it gains.
+int64_t attention_ws_bound(int64_t wgs, int64_t nk, int64_t slots, int qpb) {
+  const int64_t rem = slots > 0 ? wgs % slots : 0;
+  const int k = rem ? split_candidate(rem, nk, slots) : 1;
+  return k > 1 ? rem * k * qpb * (kAD + 2) * (int64_t)sizeof(float) : 0;
 }
 int64_t attention_ws_bytes(const AttnPlan& p, int qpb) { return p.units * qpb * (kAD + 2) * (int64_t)sizeof(float); }
 
@@ -1433,11 +1508,12 @@ int attention_run(const void* q, const int64_t q_strides[3], const void* k, cons
   if (nqb > INT32_MAX || wgs > UINT32_MAX / 8) return unsupported("too many query blocks");
   a.nqb = (int)nqb;
   a.qpb = cfg.qpb;
-  AttnPlan plan{wgs, wgs, 0, 1};
+  AttnPlan plan{wgs, wgs, 0, 1, 0.0};
   if (workspace_bytes > 0) {
-    plan = attention_plan(wgs, nk, attention_slots(kern));
-    if (attention_ws_bytes(plan, cfg.qpb) > workspace_bytes)
+    const int64_t slots = attention_slots(kern);
+    if (attention_ws_bound(wgs, nk, slots, cfg.qpb) > workspace_bytes)
       return fail("workspace smaller than oga_attention_workspace_bytes");
+    plan = attention_plan(kern, wgs, nk, slots);
   }
   a.nfull = plan.nfull;
   a.ksplit = plan.ksplit;
@@ -1504,26 +1580,35 @@ int attention_fp8_run(const void* q, const int64_t q_strides[3], const void* k, 
   a.vt = (const uint8_t*)workspace;
   a.vt_npad = (nk + kAK - 1) / kAK * kAK;
   a.q_ds = q_descale; a.k_ds = k_descale; a.v_ds = v_descale;
-  const int64_t nqb = (nq + kF8Q - 1) / kF8Q;
+  // (bounds with the narrow form's query blocks, the larger number)
+  constexpr int kMinQ = F8Cfg<kF8Narrow>::kQ;
+  if ((nq + kMinQ - 1) / kMinQ > INT32_MAX || (nq + kMinQ - 1) / kMinQ * heads * batch > UINT32_MAX / 8)
+    return unsupported("too many query blocks");
+  AttnPlan plan{};
+  const AttnKernel kern = fp8_kernel(batch, nq, nk, heads, &plan);
+  const AttnCfg cfg = attn_cfg(kern);
+  const int64_t nqb = (nq + cfg.qpb - 1) / cfg.qpb;
   const int64_t wgs = nqb * heads * batch;
-  if (nqb > INT32_MAX || wgs > UINT32_MAX / 8) return unsupported("too many query blocks");
   a.nqb = (int)nqb;
-  a.qpb = kF8Q;
-  AttnPlan plan = attention_plan(wgs, nk, attention_slots(kFp8));
-  if (vtb + attention_ws_bytes(plan, kF8Q) > workspace_bytes) plan = AttnPlan{wgs, wgs, 0, 1};
+  a.qpb = cfg.qpb;
+  if (vtb + attention_ws_bytes(plan, cfg.qpb) > workspace_bytes) plan = AttnPlan{wgs, wgs, 0, 1, 0.0};
   a.nfull = plan.nfull;
   a.ksplit = plan.ksplit;
   a.part_o = plan.units ? (float*)((char*)workspace + vtb) : nullptr;
-  a.part_ml = plan.units ? a.part_o + plan.units * kF8Q * kAD : nullptr;
+  a.part_ml = plan.units ? a.part_o + plan.units * cfg.qpb * kAD : nullptr;
   a.xcd_remap = plan.nfull % 8 == 0;
   hipStream_t st = (hipStream_t)stream;
   hipLaunchKernelGGL(k_fp8_v_transpose, dim3((unsigned)(a.vt_npad / kAK), (unsigned)heads, (unsigned)batch), dim3(256),
                      0, st, (const uint8_t*)v, a.v_sb, a.v_sn, a.v_sh, (uint8_t*)workspace, nk, a.vt_npad, (int)heads);
   int rc = launch_status();
   if (rc) return rc;
-  hipLaunchKernelGGL(k_attention_fp8, dim3((unsigned)(plan.nfull + plan.units)), dim3(64 * kF8W), 0, st, a);
+  const dim3 grid((unsigned)(plan.nfull + plan.units));
+  if (kern == kFp8Wide)
+    hipLaunchKernelGGL(k_attention_fp8<kF8Wide>, grid, dim3(cfg.threads), 0, st, a);
+  else
+    hipLaunchKernelGGL(k_attention_fp8<kF8Narrow>, grid, dim3(cfg.threads), 0, st, a);
   if (plan.units) {
-    const int64_t rows = (wgs - plan.nfull) * kF8Q;
+    const int64_t rows = (wgs - plan.nfull) * cfg.qpb;
     hipLaunchKernelGGL(k_attention_combine, dim3((unsigned)((rows * (kAD / 8) + 255) / 256)), dim3(256), 0, st, a,
                        rows);
   }
@@ -1546,7 +1631,7 @@ extern "C" int64_t oga_attention_workspace_bytes(int64_t batch, int64_t nq, int6
   const int qpb = attn_cfg(kern).qpb;
   const int64_t nqb = (nq + qpb - 1) / qpb;
   if (nqb > INT32_MAX || heads > INT32_MAX || nqb * heads > (int64_t)(UINT32_MAX / 8) / batch) return 0;
-  return attention_ws_bytes(attention_plan(nqb * heads * batch, nk, attention_slots(kern)), qpb);
+  return attention_ws_bound(nqb * heads * batch, nk, attention_slots(kern), qpb);
 }
 
 extern "C" int oga_attention_ws(const void* q, const int64_t q_strides[3], const void* k, const int64_t k_strides[3],
@@ -1571,10 +1656,11 @@ extern "C" int oga_attention_e4m3_out_ws(const void* q, const int64_t q_strides[
 extern "C" int64_t oga_attention_fp8_workspace_bytes(int64_t batch, int64_t nq, int64_t nk, int64_t heads,
                                                      int64_t head_dim) {
   if (batch <= 0 || nq <= 0 || nk <= 0 || heads <= 0 || head_dim != kAD) return 0;
-  const int64_t nqb = (nq + kF8Q - 1) / kF8Q;
-  if (nqb > INT32_MAX || heads > 65535 || batch > 65535) return 0;
-  return vt_bytes(batch, heads, nk) +
-         attention_ws_bytes(attention_plan(nqb * heads * batch, nk, attention_slots(kFp8)), kF8Q);
+  constexpr int kMinQ = F8Cfg<kF8Narrow>::kQ;
+  if ((nq + kMinQ - 1) / kMinQ > INT32_MAX || heads > 65535 || batch > 65535) return 0;
+  AttnPlan plan{};
+  const AttnKernel kern = fp8_kernel(batch, nq, nk, heads, &plan);
+  return vt_bytes(batch, heads, nk) + attention_ws_bytes(plan, attn_cfg(kern).qpb);
 }
 
 extern "C" int oga_attention_fp8_ws(const void* q8, const int64_t q_strides[3], const void* k8,

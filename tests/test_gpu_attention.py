@@ -275,6 +275,31 @@ def test_fp8_attention_kernel(b, nq, nk, h):
     _check_fp8(out.float().cpu().numpy(), ref, _fp8_rounding_bound(qe, ke, ve), f"fp8 kernel {b}x{nq}x{nk}x{h}")
 
 
+@pytest.mark.parametrize("b,nq,nk,h", [(1, 1, 1, 8), (1, 127, 63, 8), (2, 128, 64, 8), (1, 129, 65, 8), (1, 385, 193, 8),
+                                       (1, 256, 2113, 8),   # 16 workgroups, 34 key steps: key parts and their merge
+                                       (1, 4480, 300, 8)])  # more workgroups than one per CU
+def test_fp8_attention_narrow_form_edges(b, nq, nk, h):
+    """The FP8 kernel's 4-wave form at the edges of its 128-query blocks and
+    64-key steps, with a partial last step, with its key-split parts and with
+    several workgroups per CU, against float64 attention at the e4m3 bars (a
+    single output row or two have no RMS to speak of: the element bound alone)."""
+    from opengenie_amd.attention import flash_attn_func
+    from opengenie_amd.ltx_ops import fused_fp8_quantize_e4m3_per_head_4d
+
+    q, k, v = (randn((b, n, h, 128), 970 + i + n).to(DEV) for i, n in enumerate((nq, nk, nk)))
+    (q8, qs), (k8, ks), (v8, vs) = (fused_fp8_quantize_e4m3_per_head_4d(t) for t in (q, k, v))
+    out = flash_attn_func(q8, k8, v8, q_descale=qs, k_descale=ks, v_descale=vs)
+    torch.cuda.synchronize()
+    _ran("flash_attn_func_fp8")
+    qe, ke, ve = (_fp8_exact(t, s) for t, s in ((q8, qs), (k8, ks), (v8, vs)))
+    ref = O.attention(*[np.ascontiguousarray(x.transpose(0, 2, 1, 3)) for x in (qe, ke, ve)]).transpose(0, 2, 1, 3)
+    got, bound = out.float().cpu().numpy(), _fp8_rounding_bound(qe, ke, ve)
+    if nq * h >= 128:
+        _check_fp8(got, ref, bound, f"fp8 narrow b{b} nq{nq} nk{nk} h{h}")
+    else:
+        assert (np.abs(got - ref) <= (1 + 2.0 ** -6) * bound + 2.0 ** -8 * np.abs(ref) + 1e-6).all()
+
+
 def test_fp8_attention_key_split():
     """17 query blocks x 16 heads = 272 workgroups of the FP8 kernel: on a
     256-CU device the 16 past the whole round run as key parts merged by the
