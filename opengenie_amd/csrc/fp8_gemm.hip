@@ -32,8 +32,9 @@
 //
 // Two kernels share this loop: k_fp8_gemm_ring (K >= 256, N % 128 == 0, bf16
 // or no bias) is persistent, one workgroup per CU looping over tiles with
-// the slab ring running on across tile boundaries; k_fp8_gemm (every other
-// supported shape) runs one workgroup per tile.
+// the slab ring running on across tile boundaries, and is built for six
+// tiles from 256 x 256 down to 64 x 128 (choose_tile); k_fp8_gemm (every
+// other supported shape) runs one workgroup per 256 x 256 tile.
 //
 // LDS layout of an operand slab (256 rows x 128 bytes): two rows share one
 // 256-byte line of the 64 LDS banks; row r's 16-byte chunk c (c = 0..7)
@@ -51,6 +52,8 @@
 // block in LDS and writes whole rows, so HBM sees full lines.
 // Workgroups are numbered so that the eight XCDs (which receive workgroups
 // round-robin) each own a contiguous, M-grouped range of tiles.
+#include <utility>
+
 #include "common.h"
 #include "host.h"
 
@@ -524,7 +527,6 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
 // waited for here; the next tile's first odd step waits for them with the
 // DMA sent before them.
 constexpr int kStagePitch = 136;  // bytes per staged row of 64 bf16 columns
-static_assert(32 * kStagePitch <= kSlabBytes / kWaves, "a staging pass fits the wave's quarter of an A buffer");
 // Staged row r, 16-byte chunk c (of 8) sits at byte r * kStagePitch + 16c.
 // Writes: lane (fr, fh) stores 8 bytes of row fr at chunk c, half fh; each
 // 32-lane half of a ds_write_b64 must touch 64 distinct banks. Reads: lane l
@@ -599,18 +601,60 @@ __device__ const uint16_t kNegZeroRow[128] = {
 #undef OGA_NZ8
 };
 
-template <bool PARTIAL, bool O16>
+// f(IC<0>{}), ..., f(IC<N-1>{}).
+template <typename F, int... I>
+OGA_DEVICE void unroll_seq(F&& f, std::integer_sequence<int, I...>) {
+  (f(IC<I>{}), ...);
+}
+template <int N, typename F>
+OGA_DEVICE void unroll(F&& f) {
+  unroll_seq(f, std::make_integer_sequence<int, N>{});
+}
+
+// Tile of the persistent kernel: 64 JB rows x 64 IB columns, JB x IB blocks
+// of 32 x 32 per wave. A slab of a smaller tile is consumed sooner, so its
+// DMA is sent more slabs ahead (kAhead), as far as LDS holds them.
+template <int IB, int JB>
+struct RingTile {
+  static_assert((IB == 2 && JB >= 1 && JB <= 3) || (IB == 4 && JB >= 2 && JB <= 4), "supported tiles");
+  static constexpr int kBM = 64 * JB, kBN = 64 * IB;
+  static constexpr int kASlab = kBM * GKS, kWSlab = kBN * GKS;
+  static constexpr int kAhead = IB == 2 ? 6 - JB : JB == 2 ? 3 : 2;
+  static constexpr int kABufs = kAhead + 1, kWBufs = kAhead;
+  static constexpr int kWOff = kABufs * kASlab;             // W buffers after the A buffers
+  static constexpr int kRing = kWOff + kWBufs * kWSlab;
+  static constexpr int kADma = 2 * JB, kWDma = 2 * IB;      // 1 KiB DMA instructions per wave and slab
+  static constexpr int kGroup = 32 / JB;                    // M-group of ~2048 rows
+  // Epilogue staging (32 rows x 64 columns per wave and pass): padded rows
+  // after the ring where they fit, else in the wave's quarter of the A buffer
+  // of the tile's last slab, padded or (quarters of 4 KiB) swizzled.
+  static constexpr bool kStageApart = kRing + kWaves * 32 * kStagePitch <= 160 * 1024;
+  static constexpr bool kStagePacked = !kStageApart && kASlab / kWaves < 32 * kStagePitch;
+  static constexpr int kPitch = kStagePacked ? 128 : kStagePitch;
+  static constexpr int kStageWave = 32 * kPitch;
+  static constexpr int kLds = kStageApart ? kRing + kWaves * kStageWave : kRing;
+  static_assert(kLds <= 160 * 1024, "LDS budget");
+  static_assert(kStageApart || kStageWave <= kASlab / kWaves, "a staging pass fits the wave's quarter");
+  // In flight at the wait for slab d + 1: A of slabs d + 2 .. d + kAhead and
+  // W of d + 2 .. d + kAhead - 1.
+  static constexpr int kInFlight = (kAhead - 1) * kADma + (kAhead - 2) * kWDma;
+  static_assert(kInFlight < 64 && (kAhead - 1) * (kADma + kWDma) < 64, "vmcnt range");
+};
+
+template <int IB, int JB, bool PARTIAL, bool O16>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1))) void k_fp8_gemm_ring(
     GemmArgs g) {
-  __shared__ uint4 smem[(kABufs + kWBufs) * kSlabBytes / 16];
+  using T = RingTile<IB, JB>;
+  static_assert(!PARTIAL || (IB == 4 && JB == 4), "K-chunks are cut from 256 x 256 tiles");
+  __shared__ uint4 smem[T::kLds / 16];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
   const int wm = wv >> 1, wn = wv & 1;
   const int fr = lane & 31, fh = lane >> 5;
-  const int per_group = kGroupM * g.tiles_n;
-  const int nslab = g.k / GKS;  // >= 2
+  const int per_group = T::kGroup * g.tiles_n;
+  const int nslab = g.k / GKS;  // >= kAhead
   uint8_t* lds_bytes = (uint8_t*)smem;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void*)smem;
 
@@ -634,10 +678,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
       kn = g.kchunk;
     }
     const int grp = t / per_group;
-    const int first_m = grp * kGroupM;
-    const int gsize = min(g.tiles_m - first_m, kGroupM);
-    m0 = (first_m + (t % per_group) % gsize) * GM;
-    n0 = ((t % per_group) / gsize) * GN;
+    const int first_m = grp * T::kGroup;
+    const int gsize = min(g.tiles_m - first_m, T::kGroup);
+    m0 = (first_m + (t % per_group) % gsize) * T::kBM;
+    n0 = ((t % per_group) / gsize) * T::kBN;
   };
   // The operands are read through buffer resources based at the tile's first
   // row and sized to its rows inside the matrix: a DMA lane past the edge is
@@ -651,21 +695,21 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
                      __builtin_amdgcn_readfirstlane((int)bytes), kBufferWord3};
     return r;
   };
-  auto rsrc = [&](const uint8_t* base, int r0, int rows, int64_t ld) {
+  auto rsrc = [&](const uint8_t* base, int r0, int rows, int tile_rows, int64_t ld) {
     // < 2^32 bytes: 256 * ld + K fits (host check)
-    return resource(base + (int64_t)r0 * ld, (uint32_t)(min(rows - r0, GM) * ld));
+    return resource(base + (int64_t)r0 * ld, (uint32_t)(min(rows - r0, tile_rows) * ld));
   };
   // DMA instructions i and i + 2 of a wave cover rows 16 apart at the same
   // chunk (their line indices differ by 8), so two per-lane offsets per
-  // operand serve all eight: instruction i reads row row_(i%2) + 16*(i/2).
+  // operand serve all of them: instruction i reads row row_(i%2) + 16*(i/2).
   uint32_t a_off[2], w_off[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int line = (wv * kDmaPerOp + i) * 4 + (lane >> 4);
-    const int c16 = (lane & 15) ^ (line & 7);
-    const int row = 2 * line + (c16 >> 3);
-    a_off[i] = (uint32_t)(row * g.lda + (c16 & 7) * 16);
-    w_off[i] = (uint32_t)(row * g.ldw + (c16 & 7) * 16);
+    const int sub = i * 4 + (lane >> 4);  // line within the wave's part (a multiple of 8 lines)
+    const int c16 = (lane & 15) ^ (sub & 7);
+    const int row = 2 * sub + (c16 >> 3);
+    a_off[i] = (uint32_t)((wv * 8 * T::kADma + row) * g.lda + (c16 & 7) * 16);
+    w_off[i] = (uint32_t)((wv * 8 * T::kWDma + row) * g.ldw + (c16 & 7) * 16);
   }
   const uint32_t a_row16 = (uint32_t)(16 * g.lda), w_row16 = (uint32_t)(16 * g.ldw);
   // DMA instruction I of operand A or W for k-slab dk through resource rs
@@ -674,111 +718,113 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   auto dma = [&](auto i_c, auto w_c, const i32x4& rs, uint32_t buf, int dk) {
     constexpr int I = decltype(i_c)::value;
     constexpr bool W = decltype(w_c)::value;
-    const int blk = wv * kDmaPerOp + I;
+    const int blk = wv * (W ? T::kWDma : T::kADma) + I;
     const uint32_t voff = W ? w_off[I & 1] + (I >> 1) * w_row16 : a_off[I & 1] + (I >> 1) * a_row16;
     buffer_load_lds(rs, (lds_void*)(lds_bytes + buf + blk * 1024), 16, (int)voff, dk * GKS, 0, 0);
   };
   auto issue_all = [&](auto w_c, const i32x4& rs, uint32_t buf, int dk) {
-    dma(IC<0>{}, w_c, rs, buf, dk); dma(IC<1>{}, w_c, rs, buf, dk); dma(IC<2>{}, w_c, rs, buf, dk);
-    dma(IC<3>{}, w_c, rs, buf, dk); dma(IC<4>{}, w_c, rs, buf, dk); dma(IC<5>{}, w_c, rs, buf, dk);
-    dma(IC<6>{}, w_c, rs, buf, dk); dma(IC<7>{}, w_c, rs, buf, dk);
+    unroll<decltype(w_c)::value ? T::kWDma : T::kADma>([&](auto i_c) { dma(i_c, w_c, rs, buf, dk); });
   };
-  // Ring position s (counted across tiles): A slab in A buffer s % 3, W slab
-  // in W buffer s % 2.
-  auto abuf = [&](int s) { return (uint32_t)((s % kABufs) * kSlabBytes); };
-  auto wbuf = [&](int s) { return (uint32_t)(kWBase + (s % kWBufs) * kSlabBytes); };
+  // Ring position s (counted across tiles): A slab in A buffer s % kABufs, W
+  // slab in W buffer s % kWBufs.
+  auto abuf = [&](int s) { return (uint32_t)((s % T::kABufs) * T::kASlab); };
+  auto wbuf = [&](int s) { return (uint32_t)(T::kWOff + (s % T::kWBufs) * T::kWSlab); };
 
-  // Fragment bases (as in k_fp8_gemm); the A bases are the W bases plus the
-  // uniform (wm - wn) * 16 KiB, added with the slab buffer offset.
+  // Fragment bases (as in k_fp8_gemm, the wave's W blocks IB wn + i, its A
+  // blocks JB wm + j, 4 KiB each); the A bases are the W bases plus a
+  // uniform difference, added with the slab buffer offset.
   uint32_t lw[2][2];
 #pragma unroll
   for (int p = 0; p < 2; ++p)
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
       const uint32_t in_line = (fr >> 1) * 256 + (8 * (fr & 1) + ((4 * p + 2 * fh + q) ^ ((fr >> 1) & 7))) * 16;
-      lw[p][q] = lds0 + wn * 16384 + in_line;
+      lw[p][q] = lds0 + wn * (IB * 4096) + in_line;
     }
-  const uint32_t a_minus_w = (uint32_t)((wm - wn) * 16384);
+  const uint32_t a_minus_w = (uint32_t)((wm * JB - wn * IB) * 4096);
 
-  f32x16 acc[4][4];
+  f32x16 acc[IB][JB];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < IB; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < JB; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-#define OGA_FRAG_W(P, i) frag<(i) * 4096>(lw[P][0] + wb, lw[P][1] + wb)
-#define OGA_FRAG_A(P, j) frag<(j) * 4096>(lw[P][0] + ab, lw[P][1] + ab)
-// MFMA of block (i, j); the first step of a tile (Z) starts from zero.
-#define OGA_MF(i, j) acc[i][j] = mfma(cw[i], ca[j], Z ? kZero16 : acc[i][j])
-  // Even step of ring slab s: as in k_fp8_gemm, with the A DMA of k-slab dk
-  // through resource rs into ring slot s + 2; on a tile's first slab (z_c)
-  // the MFMAs take zero accumulators.
-  const f32x16 kZero16 = {};
-  auto even_step = [&](auto z_c, int s, int dk, const i32x4& rs, i32x8(&cw)[4], i32x8(&ca)[4], i32x8(&nw)[4],
-                       i32x8(&na)[4]) {
-    constexpr bool Z = decltype(z_c)::value;
-    const uint32_t ab = abuf(s) + a_minus_w, wb = wbuf(s), an = abuf(s + 2);
-    OGA_MF(0, 0); nw[0] = OGA_FRAG_W(1, 0); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(0, 1); nw[1] = OGA_FRAG_W(1, 1); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(0, 2); nw[2] = OGA_FRAG_W(1, 2); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(0, 3); nw[3] = OGA_FRAG_W(1, 3); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(1, 0); na[0] = OGA_FRAG_A(1, 0); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(1, 1); na[1] = OGA_FRAG_A(1, 1); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(1, 2); na[2] = OGA_FRAG_A(1, 2); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(1, 3); na[3] = OGA_FRAG_A(1, 3); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(2, 0); dma(IC<0>{}, IC<0>{}, rs, an, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(2, 1); dma(IC<1>{}, IC<0>{}, rs, an, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(2, 2); dma(IC<2>{}, IC<0>{}, rs, an, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(2, 3); dma(IC<3>{}, IC<0>{}, rs, an, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(3, 0); dma(IC<4>{}, IC<0>{}, rs, an, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(3, 1); dma(IC<5>{}, IC<0>{}, rs, an, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(3, 2); dma(IC<6>{}, IC<0>{}, rs, an, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(3, 3); dma(IC<7>{}, IC<0>{}, rs, an, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_LGKM_WAIT(0, "+v"(nw[0]), "+v"(nw[1]), "+v"(nw[2]), "+v"(nw[3]), "+v"(na[0]), "+v"(na[1]), "+v"(na[2]),
-                  "+v"(na[3]));
+  // Fragment F of step parity P from the slab buffers at byte offsets ab (A)
+  // and wb (W): W block F, then A block F - IB.
+  auto read_frag = [&](auto p_c, auto f_c, uint32_t ab, uint32_t wb, i32x8(&nw)[IB], i32x8(&na)[JB]) {
+    constexpr int P = decltype(p_c)::value, F = decltype(f_c)::value;
+    if constexpr (F < IB)
+      nw[F] = frag<F * 4096>(lw[P][0] + wb, lw[P][1] + wb);
+    else
+      na[F - IB] = frag<(F - IB) * 4096>(lw[P][0] + ab, lw[P][1] + ab);
   };
-  // Odd step of ring slab s: wait for slab s + 1 (only the A DMA of the even
-  // step may stay in flight; every older DMA, bias load and output store is
-  // waited for), barrier, MFMAs with the fragments of slab s + 1 read between
-  // the first eight, and the W DMA of k-slab dk through resource rs into
-  // ring slot s + 2.
-  auto odd_step = [&](int s, int dk, const i32x4& rs, i32x8(&cw)[4], i32x8(&ca)[4], i32x8(&nw)[4],
-                      i32x8(&na)[4]) {
-    constexpr bool Z = false;
-    const uint32_t ab = abuf(s + 1) + a_minus_w, wb = wbuf(s + 1), wn2 = wbuf(s + 2);
-    OGA_WAIT_VM(kDmaPerOp);
+  // The fragments read since the last wait are there: the wait, then every
+  // fragment named after it (volatile, so in this order), so that no use of
+  // them can be scheduled before it.
+  auto wait_frags = [&](i32x8(&nw)[IB], i32x8(&na)[JB]) {
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(nw[0]), "+v"(na[0]));
+#pragma unroll
+    for (int i = 1; i < IB; ++i) asm volatile("" : "+v"(nw[i]));
+#pragma unroll
+    for (int j = 1; j < JB; ++j) asm volatile("" : "+v"(na[j]));
+  };
+  // One 64-byte K step: its IB x JB MFMAs (Z: from zero accumulators, a
+  // tile's first step), with the IB + JB fragment reads of the next step and
+  // then this step's DMA instructions (of operand W or A: k-slab dk through
+  // resource rs into buffer `buf`) spread evenly between them.
+  const f32x16 kZero16 = {};
+  auto step = [&](auto z_c, auto p_c, auto w_c, uint32_t ab, uint32_t wb, uint32_t buf, int dk, const i32x4& rs,
+                  i32x8(&cw)[IB], i32x8(&ca)[JB], i32x8(&nw)[IB], i32x8(&na)[JB]) {
+    constexpr bool Z = decltype(z_c)::value;
+    constexpr int R = IB + JB, D = decltype(w_c)::value ? T::kWDma : T::kADma, NM = IB * JB;
+    unroll<NM>([&](auto n_c) {
+      constexpr int N = decltype(n_c)::value, i = N / JB, j = N % JB;
+      acc[i][j] = mfma(cw[i], ca[j], Z ? kZero16 : acc[i][j]);
+      unroll<R>([&](auto f_c) {
+        if constexpr (decltype(f_c)::value * NM / (R + D) == N) read_frag(p_c, f_c, ab, wb, nw, na);
+      });
+      unroll<D>([&](auto d_c) {
+        if constexpr ((R + decltype(d_c)::value) * NM / (R + D) == N) dma(d_c, w_c, rs, buf, dk);
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    wait_frags(nw, na);
+  };
+  // Even step of ring slab s: as in k_fp8_gemm, with the A DMA of k-slab dk
+  // through resource rs into ring slot s + kAhead (the A buffer of slab
+  // s - 1, released by the barrier before); on a tile's first slab (z_c)
+  // the MFMAs take zero accumulators.
+  auto even_step = [&](auto z_c, int s, int dk, const i32x4& rs, i32x8(&cw)[IB], i32x8(&ca)[JB], i32x8(&nw)[IB],
+                       i32x8(&na)[JB]) {
+    step(z_c, IC<1>{}, IC<0>{}, abuf(s) + a_minus_w, wbuf(s), abuf(s + T::kAhead), dk, rs, cw, ca, nw, na);
+  };
+  // Odd step of ring slab s: wait for slab s + 1 (only the DMA sent after it
+  // may stay in flight; bias loads and output stores among the newest count
+  // as part of it, which only waits for more), barrier, MFMAs with the
+  // fragments of slab s + 1 read between them, and the W DMA of k-slab dk
+  // through resource rs into ring slot s + kAhead (slab s's W buffer).
+  auto odd_step = [&](int s, int dk, const i32x4& rs, i32x8(&cw)[IB], i32x8(&ca)[JB], i32x8(&nw)[IB],
+                      i32x8(&na)[JB]) {
+    OGA_WAIT_VM(T::kInFlight);
     OGA_BARRIER();
     __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(0, 0); nw[0] = OGA_FRAG_W(0, 0); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(0, 1); nw[1] = OGA_FRAG_W(0, 1); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(0, 2); nw[2] = OGA_FRAG_W(0, 2); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(0, 3); nw[3] = OGA_FRAG_W(0, 3); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(1, 0); na[0] = OGA_FRAG_A(0, 0); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(1, 1); na[1] = OGA_FRAG_A(0, 1); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(1, 2); na[2] = OGA_FRAG_A(0, 2); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(1, 3); na[3] = OGA_FRAG_A(0, 3); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(2, 0); dma(IC<0>{}, IC<1>{}, rs, wn2, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(2, 1); dma(IC<1>{}, IC<1>{}, rs, wn2, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(2, 2); dma(IC<2>{}, IC<1>{}, rs, wn2, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(2, 3); dma(IC<3>{}, IC<1>{}, rs, wn2, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(3, 0); dma(IC<4>{}, IC<1>{}, rs, wn2, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(3, 1); dma(IC<5>{}, IC<1>{}, rs, wn2, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(3, 2); dma(IC<6>{}, IC<1>{}, rs, wn2, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_MF(3, 3); dma(IC<7>{}, IC<1>{}, rs, wn2, dk); __builtin_amdgcn_sched_barrier(0);
-    OGA_LGKM_WAIT(0, "+v"(nw[0]), "+v"(nw[1]), "+v"(nw[2]), "+v"(nw[3]), "+v"(na[0]), "+v"(na[1]), "+v"(na[2]),
-                  "+v"(na[3]));
+    step(IC<0>{}, IC<0>{}, IC<1>{}, abuf(s + 1) + a_minus_w, wbuf(s + 1), wbuf(s + T::kAhead), dk, rs, cw, ca, nw, na);
   };
-#undef OGA_MF
 
   // Staging: a pass holds 32 rows x 64 columns of the wave's block (block
   // row j, column half h) inside the wave's 8 KiB quarter. Lane (fr, fh)
   // writes at sw + 64*(i - 2h) + 16q; lane l reads its row (srow, plus 4u)
   // at sr + 4u * kStagePitch.
-  const int srow = (lane >> 4) + 16 * ((lane >> 3) & 1);
-  const uint32_t sw = (uint32_t)(fr * kStagePitch + fh * 8);
-  const uint32_t sr = (uint32_t)(srow * kStagePitch + (lane & 7) * 16);
+  // Swizzled (packed) rows keep chunk c of row r at c ^ ((r / 2) % 8), and a
+  // read covers eight consecutive rows: the two rows of a 16-lane group then
+  // lie in different halves of the banks.
+  constexpr int kRowStep = T::kStagePacked ? 8 : 4;  // rows from one read of a lane to its next
+  const int srow = T::kStagePacked ? lane >> 3 : (lane >> 4) + 16 * ((lane >> 3) & 1);
+  const uint32_t sw = (uint32_t)(fr * T::kPitch + fh * 8);
+  const uint32_t sr = (uint32_t)(srow * T::kPitch + (T::kStagePacked ? 0 : (lane & 7) * 16));
+  const int swz_w = T::kStagePacked ? (fr >> 1) & 7 : 0;
 
   // sa * sb of each group, read before any DMA is in flight (read in the
   // epilogue, they would make it wait for every outstanding DMA).
@@ -794,31 +840,19 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   // W of the group holding columns n0 .. n0 + 255, from its first row.
   auto wrsrc = [&](int n0) {
     const int gi = n0 / g.group_n, r0 = n0 - gi * g.group_n;
-    return rsrc(pick(g.wg, gi), r0, g.group_n, g.ldw);
+    return rsrc(pick(g.wg, gi), r0, g.group_n, T::kBN, g.ldw);
   };
-  i32x4 ra = rsrc(g.a, m0, g.m, g.lda), rw = wrsrc(n0);
-  issue_all(IC<0>{}, ra, abuf(0), kb);
-  issue_all(IC<1>{}, rw, wbuf(0), kb);
-  issue_all(IC<0>{}, ra, abuf(1), kb + 1);
-  issue_all(IC<1>{}, rw, wbuf(1), kb + 1);
-  OGA_WAIT_VM(2 * kDmaPerOp);
+  i32x4 ra = rsrc(g.a, m0, g.m, T::kBM, g.lda), rw = wrsrc(n0);
+  unroll<T::kAhead>([&](auto d_c) {
+    constexpr int D = decltype(d_c)::value;
+    issue_all(IC<0>{}, ra, abuf(D), kb + D);
+    issue_all(IC<1>{}, rw, wbuf(D), kb + D);
+  });
+  OGA_WAIT_VM((T::kAhead - 1) * (T::kADma + T::kWDma));
   OGA_BARRIER();
-  i32x8 xw[4], xa[4], yw[4], ya[4];
-  {
-    const uint32_t ab = abuf(0) + a_minus_w, wb = wbuf(0);
-    xw[0] = OGA_FRAG_W(0, 0);
-    xw[1] = OGA_FRAG_W(0, 1);
-    xw[2] = OGA_FRAG_W(0, 2);
-    xw[3] = OGA_FRAG_W(0, 3);
-    xa[0] = OGA_FRAG_A(0, 0);
-    xa[1] = OGA_FRAG_A(0, 1);
-    xa[2] = OGA_FRAG_A(0, 2);
-    xa[3] = OGA_FRAG_A(0, 3);
-  }
-#undef OGA_FRAG_W
-#undef OGA_FRAG_A
-  OGA_LGKM_WAIT(0, "+v"(xw[0]), "+v"(xw[1]), "+v"(xw[2]), "+v"(xw[3]), "+v"(xa[0]), "+v"(xa[1]), "+v"(xa[2]),
-                "+v"(xa[3]));
+  i32x8 xw[IB], xa[JB], yw[IB], ya[JB];
+  unroll<IB + JB>([&](auto f_c) { read_frag(IC<0>{}, f_c, abuf(0) + a_minus_w, wbuf(0), xw, xa); });
+  wait_frags(xw, xa);
 
   for (;;) {
     // The next unit (after the last one: this unit again, whose first slabs
@@ -827,34 +861,37 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     const bool more = vn < g.units;
     int nm0, nn0, nkb, nkn, nsp;
     unit(more ? vn : v, nm0, nn0, nkb, nkn, nsp);
-    const i32x4 nra = rsrc(g.a, nm0, g.m, g.lda), nrw = wrsrc(nn0);
+    const i32x4 nra = rsrc(g.a, nm0, g.m, T::kBM, g.lda), nrw = wrsrc(nn0);
     // The group of this tile: its bias, output, scale and first column.
     const int gi = n0 / g.group_n, nc0 = n0 - gi * g.group_n;
     const void* const gbias = pick(g.biasg, gi);
     // Bias of the 16 columns this lane stores, (lane % 8) * 8 + 0..7 of each
     // 64-column half of the wave's block, as bf16 (R(bias)). A block wholly
-    // past N reads the last 128 columns instead (its results are not
+    // past N reads the last 32 IB columns instead (its results are not
     // stored); without a bias the values are -0.0, which an add leaves every
-    // value (signed zeros included) as it is. Loaded at the tile's start;
-    // the wait of the first odd step covers them.
-    u32x4 bq[2];
+    // value (signed zeros included) as it is. Loaded at the tile's start; the
+    // wait of the first odd step covers them, or, with more than two slabs
+    // in flight, the one before the epilogue.
+    u32x4 bq[IB / 2];
     if constexpr (!PARTIAL) {
-      gu16* const bsrc = gbias ? (gu16*)gbias + min(nc0 + wn * 128, g.group_n - 128) : (gu16*)kNegZeroRow;
-      bq[0] = load_x4_unwaited((gu32x4*)(bsrc + (lane & 7) * 8));
-      bq[1] = load_x4_unwaited((gu32x4*)(bsrc + 64 + (lane & 7) * 8));
+      gu16* const bsrc = gbias ? (gu16*)gbias + min(nc0 + wn * 32 * IB, g.group_n - 32 * IB) : (gu16*)kNegZeroRow;
+#pragma unroll
+      for (int h = 0; h < IB / 2; ++h) bq[h] = load_x4_unwaited((gu32x4*)(bsrc + 64 * h + (lane & 7) * 8));
     }
-    // All slabs of the unit; the DMA of its last two fetches the first two
+    // All slabs of the unit; the DMA of its last kAhead fetches the first
     // slabs of the next unit.
     // The first slab's MFMAs start from zero accumulators.
     auto slab = [&](auto z_c, int d) {
-      const bool here = d + 2 < kn;
-      const int dk = here ? kb + d + 2 : nkb + d + 2 - kn;
+      const bool here = d + T::kAhead < kn;
+      const int dk = here ? kb + d + T::kAhead : nkb + d + T::kAhead - kn;
       even_step(z_c, s, dk, here ? ra : nra, xw, xa, yw, ya);
       odd_step(s, dk, here ? rw : nrw, yw, ya, xw, xa);
       ++s;
     };
     slab(IC<1>{}, 0);
     for (int d = 1; d < kn; ++d) slab(IC<0>{}, d);
+    // The bias loads have landed: at least two slabs of DMA came after them.
+    if constexpr (T::kAhead > 2) OGA_WAIT_VM(2 * (T::kADma + T::kWDma));
 
     if constexpr (PARTIAL) {
       // A K-chunk of a split tile: its float32 partial sums, as each lane
@@ -871,30 +908,32 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
             pw[((i * 4 + j) * 4 + q) * 64] = p4;
           }
     } else {
-    // Epilogue of tile (m0, n0): out = R(R(acc * sc) + R(bias)). Eight
-    // passes p = 2j + h (block row j, column half h) through the wave's
-    // staging quarter of A buffer s - 1 (the tile's last slab): R(acc * sc)
+    // Epilogue of tile (m0, n0): out = R(R(acc * sc) + R(bias)). Passes
+    // p = (IB/2) j + h (block row j, 64-column part h) through the wave's
+    // staging (for tiles without room for one of its own, its quarter of A
+    // buffer s - 1, the tile's last slab): R(acc * sc)
     // is staged as bf16, read back as 16-byte row pieces, the bias added,
     // and stored. The passes overlap: pass p packs its values while the
     // reads of pass p - 1 are in flight, and finishes pass p - 1 (bias and
     // stores) while its own writes are.
-    const uint32_t stg = lds0 + abuf(s - 1) + wv * (kSlabBytes / kWaves);
+    constexpr int kHalves = IB / 2, kPasses = JB * kHalves;
+    const uint32_t stg = T::kStageApart ? lds0 + T::kRing + wv * T::kStageWave : lds0 + abuf(s - 1) + wv * (T::kASlab / kWaves);
     const float sc = pick(scg, gi);
     // The stores of block row j go through a buffer resource over its 32
     // rows inside the matrix (none for a block past N), which drops rows
-    // past M. Lane l stores row 4u + srow, columns h*64 + (lane%8)*8: the
+    // past M. Lane l stores row kRowStep u + srow, columns h*64 + (lane%8)*8: the
     // row in the lane offset, h*128 bytes as the scalar offset (a lane's 16
     // bytes end inside its row, so the range check sees the row whether or
     // not it counts the scalar offset).
-    const bool col_ok = nc0 + wn * 128 < g.group_n;
-    const int rows_left = g.m - (m0 + wm * 128);
-    uint16_t* const oblk = pick(g.outg, gi) + (int64_t)(m0 + wm * 128) * g.ldo + nc0 + wn * 128;
+    const bool col_ok = nc0 + wn * 32 * IB < g.group_n;
+    const int rows_left = g.m - (m0 + wm * 32 * JB);
+    uint16_t* const oblk = pick(g.outg, gi) + (int64_t)(m0 + wm * 32 * JB) * g.ldo + nc0 + wn * 32 * IB;
     const int olane = (srow * (int)g.ldo + (lane & 7) * 8) * 2;
-    const int orow4 = 8 * (int)g.ldo;  // bytes of 4 rows
+    const int orow = kRowStep * 2 * (int)g.ldo;  // bytes from one stored row of a lane to its next
     uint2 pk[2][4];
     u32x4 ov[4];
     auto pack = [&](auto p_c) {
-      constexpr int J = decltype(p_c)::value / 2, H = decltype(p_c)::value % 2;
+      constexpr int J = decltype(p_c)::value / kHalves, H = decltype(p_c)::value % kHalves;
 #pragma unroll
       for (int ii = 0; ii < 2; ++ii)
 #pragma unroll
@@ -909,17 +948,30 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
 #pragma unroll
       for (int ii = 0; ii < 2; ++ii)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(stg + sw), "v"(pk[ii][q]), "i"(ii * 64 + q * 16)
-                       : "memory");
+        for (int q = 0; q < 4; ++q) {
+          if constexpr (T::kStagePacked)
+            asm volatile("ds_write_b64 %0, %1" ::"v"(stg + sw + (((4 * ii + q) ^ swz_w) << 4)), "v"(pk[ii][q])
+                         : "memory");
+          else
+            asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(stg + sw), "v"(pk[ii][q]), "i"(ii * 64 + q * 16)
+                         : "memory");
+        }
     };
     auto read = [&]() {
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(ov[u]) : "v"(stg + sr), "i"(u * 4 * kStagePitch));
+      for (int u = 0; u < 4; ++u) {
+        if constexpr (T::kStagePacked)
+          asm volatile("ds_read_b128 %0, %1 offset:%2"
+                       : "=v"(ov[u])
+                       : "v"(stg + sr + ((((lane & 7) ^ ((srow >> 1) + 4 * u)) & 7) << 4)), "i"(u * kRowStep * T::kPitch));
+        else
+          asm volatile("ds_read_b128 %0, %1 offset:%2"
+                       : "=v"(ov[u])
+                       : "v"(stg + sr), "i"(u * kRowStep * T::kPitch));
+      }
     };
     auto finish = [&](auto p_c) {
-      constexpr int J = decltype(p_c)::value / 2, H = decltype(p_c)::value % 2;
+      constexpr int J = decltype(p_c)::value / kHalves, H = decltype(p_c)::value % kHalves;
       const int rows_j = col_ok ? min(max(rows_left - 32 * J, 0), 32) : 0;
       const i32x4 ro = resource(oblk + (int64_t)32 * J * g.ldo, (uint32_t)(rows_j * 2 * g.ldo));
       const u32x4 bw = bq[H];
@@ -930,7 +982,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
         for (int e = 0; e < 4; ++e)
           y[e] = pack_out<O16>(out_lo<O16>(ov[u][e]) + out_lo<O16>(bw[e]),
                                out_hi<O16>(ov[u][e]) + out_hi<O16>(bw[e]));
-        buffer_store_x4(y, ro, olane + u * orow4, H * 128, kStoreNT);
+        buffer_store_x4(y, ro, olane + u * orow, H * 128, kStoreNT);
       }
       __builtin_amdgcn_sched_barrier(0);
     };
@@ -947,15 +999,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     write();
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     read();
-    next(IC<1>{});
-    next(IC<2>{});
-    next(IC<3>{});
-    next(IC<4>{});
-    next(IC<5>{});
-    next(IC<6>{});
-    next(IC<7>{});
+    unroll<kPasses - 1>([&](auto p_c) { next(IC<decltype(p_c)::value + 1>{}); });
     OGA_LGKM_WAIT(0, "+v"(ov[0]), "+v"(ov[1]), "+v"(ov[2]), "+v"(ov[3]));
-    finish(IC<7>{});
+    finish(IC<kPasses - 1>{});
     }
     __builtin_amdgcn_sched_barrier(0);
     if (!more) break;
@@ -1132,13 +1178,78 @@ int check_args(const void* a, int64_t lda, int64_t ldw, const float* scale_a, in
   return OGA_OK;
 }
 
-// The persistent schedule: whole tiles, then (split, workspace given) the
-// K-chunks of the rest and their sums. g has its shape, operands and groups.
+// The tiles the persistent kernel is built for, the 256 x 256 one (the only
+// one with split-K) first, with the times the choice between them uses, in us:
+// a slab on a chip at most half full and on a full one (where the clock drops
+// under the MFMAs' power), and the rest of a round (first slabs, epilogue).
+// Fitted to the kernel's times over 69 shapes (64 to 9216 rows, 4096 -> 4096,
+// 4096 -> 16384 and 16384 -> 4096) with every tile forced in turn, 3 to 8 %
+// rms per tile; the tile it picks was the fastest in 67 of them and within
+// 2 % in the others.
+struct TileShape {
+  int ib, jb, ahead;  // RingTile<ib, jb>
+  void (*bf16)(GemmArgs);
+  void (*f16)(GemmArgs);
+  double slab_half, slab_full, round;
+};
+template <int IB, int JB>
+TileShape tile_shape(double slab_half, double slab_full, double round) {
+  return {IB, JB, RingTile<IB, JB>::kAhead, k_fp8_gemm_ring<IB, JB, false, false>,
+          k_fp8_gemm_ring<IB, JB, false, true>, slab_half, slab_full, round};
+}
+const TileShape kTiles[] = {
+    tile_shape<4, 4>(1.05, 1.37, 7.9), tile_shape<4, 3>(0.80, 1.03, 7.5), tile_shape<4, 2>(0.60, 0.74, 5.4),
+    tile_shape<2, 3>(0.54, 0.60, 4.1), tile_shape<2, 2>(0.41, 0.455, 2.8), tile_shape<2, 1>(0.35, 0.35, 2.3)};
+constexpr double kSplitUs = 13.7, kSplitChunkUs = 0.04;  // K-chunks and reduce: both launches, a chunk's partials
+
+// The tile with the shortest modelled time: whole rounds of the CUs, then the
+// rest as one more round or (256 x 256, workspace given) as K-chunks. What
+// decides is how the tile count meets the CU count: 1537 x 4096 outputs are
+// 112 of the 256 x 256 tiles (41 us at K = 4096) but 208 of 128 x 256 (29 us),
+// 9216 x 4096 is 2.25 rounds of the one (141 us) and exactly three of 192 x
+// 256 (122 us); 256 x 4096 runs 15 us as 128 tiles of 64 x 128, 24 us as
+// K-chunks and their sums.
+const TileShape& choose_tile(int64_t m, int64_t n, int64_t k, int64_t cus, const SplitPlan& split) {
+  const int64_t nslab = k / GKS;
+  const TileShape* best = nullptr;
+  double best_us = 0.0;
+  for (const TileShape& t : kTiles) {
+    if (nslab < t.ahead) continue;
+    const int64_t nt = ((m + 64 * t.jb - 1) / (64 * t.jb)) * ((n + 64 * t.ib - 1) / (64 * t.ib));
+    const int64_t rest = nt % cus;
+    auto slab = [&](int64_t units) {
+      const double fill = (double)units / (double)cus;
+      return t.slab_half + (t.slab_full - t.slab_half) * (fill > 0.5 ? 2.0 * fill - 1.0 : 0.0);
+    };
+    double us = (double)(nt / cus) * ((double)nslab * t.slab_full + t.round);
+    if (rest && &t == kTiles && split.split > 1)
+      us += (double)split.kchunk * slab(rest * split.split) + kSplitUs + kSplitChunkUs * (double)(rest * split.split);
+    else if (rest)
+      us += (double)nslab * slab(rest) + t.round;
+    // (5 % less than the 256 x 256 tile's: over long kernels the clock follows
+    // the MFMAs' power, and three rounds of 192 x 256 at 9216 x 16384 -> 4096,
+    // modelled 4 % shorter, measured 0.7 % longer.)
+    if (!best || us < best_us * (best == kTiles ? 0.95 : 1.0)) { best = &t; best_us = us; }
+  }
+  return *best;  // (K >= 256: the two-slab tiles always qualify)
+}
+
+void set_tiles(GemmArgs& g, int bm, int bn) {
+  g.tiles_m = (int)(((int64_t)g.m + bm - 1) / bm);
+  g.tiles_n = (int)(((int64_t)g.n + bn - 1) / bn);
+}
+
+// The persistent schedule: whole tiles, then (256 x 256 tiles, split,
+// workspace given) the K-chunks of the rest and their sums. g has its shape,
+// operands and groups.
 int launch_ring(GemmArgs& g, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
-  const int64_t nt = (int64_t)g.tiles_m * g.tiles_n;
   const int64_t cus = cu_count();
-  SplitPlan p = split_plan(g.m, (int64_t)g.tiles_n * GN, g.k, cus);
-  if (p.split > 1 && (!workspace || workspace_bytes < p.ws_bytes)) p = SplitPlan{(int)nt, 1, g.k / GKS, (int)nt, 0};
+  SplitPlan p = split_plan(g.m, g.n, g.k, cus);
+  if (p.split > 1 && (!workspace || workspace_bytes < p.ws_bytes)) p.split = 1;
+  const TileShape& tile = choose_tile(g.m, g.n, g.k, cus, p);
+  set_tiles(g, 64 * tile.jb, 64 * tile.ib);
+  const int64_t nt = (int64_t)g.tiles_m * g.tiles_n;
+  if (&tile != kTiles || p.split == 1) p = SplitPlan{(int)nt, 1, g.k / GKS, (int)nt, 0};
   g.nfull = p.nfull;
   g.split = p.split;
   g.kchunk = p.kchunk;
@@ -1146,24 +1257,19 @@ int launch_ring(GemmArgs& g, void* workspace, int64_t workspace_bytes, hipStream
   g.units = p.nfull;
   int64_t grid = g.units < cus ? g.units : cus;
   g.xcd_remap = (g.units % 8) == 0 && (grid % 8) == 0;
-  if (grid > 0) {  // none when every tile is split (fewer tiles than CUs)
-    if (g.out_f16)
-      hipLaunchKernelGGL((k_fp8_gemm_ring<false, true>), dim3((unsigned)grid), dim3(64 * kWaves), 0, stream, g);
-    else
-      hipLaunchKernelGGL((k_fp8_gemm_ring<false, false>), dim3((unsigned)grid), dim3(64 * kWaves), 0, stream, g);
-  }
+  if (grid > 0)  // none when every tile is split (fewer tiles than CUs)
+    hipLaunchKernelGGL(g.out_f16 ? tile.f16 : tile.bf16, dim3((unsigned)grid), dim3(64 * kWaves), 0, stream, g);
   if (p.split > 1) {
     g.units = p.units - p.nfull;
     grid = g.units < cus ? g.units : cus;
     g.xcd_remap = (g.units % 8) == 0 && (grid % 8) == 0;
     // the K-chunks write float32 partials (no epilogue: one instance)
-    hipLaunchKernelGGL((k_fp8_gemm_ring<true, false>), dim3((unsigned)grid), dim3(64 * kWaves), 0, stream, g);
+    hipLaunchKernelGGL((k_fp8_gemm_ring<4, 4, true, false>), dim3((unsigned)grid), dim3(64 * kWaves), 0, stream, g);
+    const dim3 reduce((unsigned)((nt - p.nfull) * kWaves));
     if (g.out_f16)
-      hipLaunchKernelGGL(k_fp8_splitk_reduce<true>, dim3((unsigned)((nt - p.nfull) * kWaves)), dim3(256), 0, stream,
-                         g);
+      hipLaunchKernelGGL(k_fp8_splitk_reduce<true>, reduce, dim3(256), 0, stream, g);
     else
-      hipLaunchKernelGGL(k_fp8_splitk_reduce<false>, dim3((unsigned)((nt - p.nfull) * kWaves)), dim3(256), 0, stream,
-                         g);
+      hipLaunchKernelGGL(k_fp8_splitk_reduce<false>, reduce, dim3(256), 0, stream, g);
   }
   return launch_status();
 }
@@ -1178,8 +1284,6 @@ void set_shape(GemmArgs& g, const void* a, int64_t lda, int64_t ldw, const float
   g.m = (int)m;
   g.n = (int)n;
   g.k = (int)k;
-  g.tiles_m = (int)((m + GM - 1) / GM);
-  g.tiles_n = (int)((n + GN - 1) / GN);
 }
 
 }  // namespace
@@ -1224,6 +1328,7 @@ extern "C" int oga_fp8_linear_dt_ws(const void* a, int64_t lda, const void* w, i
     g.group_n = g.n;
     return launch_ring(g, workspace, workspace_bytes, (hipStream_t)stream);
   }
+  set_tiles(g, GM, GN);
   const int64_t nt = (int64_t)g.tiles_m * g.tiles_n;
   g.xcd_remap = (nt % 8) == 0;
   if (g.out_f16)

@@ -786,6 +786,44 @@ def test_fp8_linear_split_k_workspace_reuse(m, n, k):
         _linear_full_check(outs[0], _device_fp8_linear(ga, gw, gsa, gsb, gb), "down-projection, split tail")
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (1, 128, 256), (65, 384, 384), (130, 640, 512),  # two, three and four slabs of K: the tiles that run so few
+    (1, 128, 640), (64, 128, 640), (65, 256, 768),   # 64 x 128 tiles: one, exact, one row more
+    (64, 65536, 640),                                # two rounds of them
+    (700, 4096, 640), (1023, 4096, 1024),            # 128 x 128
+    (1100, 4096, 1024), (1152, 16384, 512),          # 192 x 128, one round and several
+    (1537, 4096, 896),                               # 128 x 256
+    (2305, 4096, 640), (2400, 4224, 384),            # 192 x 256, and a last tile half past N
+    (6144, 4096, 256),                               # two whole rounds of them
+    (64, 4096, 8192)])                               # K-chunks
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_fp8_linear_tiles(m, n, k, dtype):
+    """The tiles of the persistent kernel at their edges (ragged rows and
+    columns, the fewest slabs of K each runs, one and several rounds of the
+    CUs) through fp8_scaled_mm, the biased output against the oracle and, bit
+    for bit, against R(unbiased + bias)."""
+    from opengenie_amd.ltx_ops import fp8_scaled_mm
+
+    x = randn((m, k), 390 + m, std=1.0)
+    sa = (x.float().abs().amax() / 448.0).reshape(())
+    a = torch.clamp(x.float() / sa, -448, 448).to(torch.float8_e4m3fn)
+    w, sb = _fp8_weights(n, k, 391 + n)
+    bias = randn((n,), 392, dtype=dtype, std=0.01)
+    ga, gw, gsa, gsb = g(a), g(w), g(sa), g(sb)
+    out = fp8_scaled_mm(ga, gw, gsa, gsb, g(bias), out_dtype=dtype)
+    nob = fp8_scaled_mm(ga, gw, gsa, gsb, None, out_dtype=dtype)
+    _ran("fp8_scaled_mm")
+    want = (nob.float() + g(bias).float()).to(dtype)
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    rows = np.unique(np.concatenate([np.arange(0, m, max(1, m // 200)), [m - 1]]))  # some rows of every tile
+    ref = O.fp8_linear(a.view(torch.uint8).numpy()[rows], w.view(torch.uint8).numpy(), float(sa), float(sb),
+                       to_T(bias), **({"out_dt": "f16"} if dtype == torch.float16 else {}))
+    got = out_np(out)[rows]
+    # bf16: 8 bits of mantissa, two roundings; fp16: the bar of test_fp8_linear_fp16_output
+    close = np.isclose(got, ref, rtol=1e-2 if dtype == torch.bfloat16 else 2e-3, atol=1e-3 * float(np.abs(ref).max()))
+    assert (~close).mean() < 1e-4, (~close).sum()
+
+
 def _bias_epilogue_ref(out_nobias: np.ndarray, bias: torch.Tensor, r=bf16_round) -> np.ndarray:
     """R(out + R(bias)): the second rounding of the FP8 linear (:1705-1709),
     R the output dtype's rounding."""
