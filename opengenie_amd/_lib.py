@@ -1,4 +1,6 @@
-"""ctypes binding of libopengenie_amd.so (the C ABI in include/opengenie_amd.h).
+"""Binding of libopengenie_amd.so (the C ABI in include/opengenie_amd.h): load()
+gives it through ctypes; call() and function() go through the compiled module
+_native, whose calls cost the wrappers less (pycall.cpp).
 
 The library is loaded on first use. If it is missing the call raises: a GPU
 tensor never silently takes another path because the extension is absent.
@@ -117,14 +119,31 @@ def available() -> bool:
     return os.path.exists(LIB_PATH)
 
 
+# ctypes makes an array type anew on every `c_int64 * n`; these are kept.
+_I64_ARRAYS = tuple(ctypes.c_int64 * n for n in range(6))
+
+
 def strides(values) -> ctypes.Array:
-    arr = (ctypes.c_int64 * len(values))(*[int(v) for v in values])
-    return arr
+    return _I64_ARRAYS[len(values)](*values)
+
+
+_fns: dict[str, object] = {}  # entry points by name, from _native where it has them
+
+
+def function(name: str):
+    fn = _fns.get(name)
+    if fn is None:
+        lib = load()
+        try:
+            from . import _native  # built with the library, linked to the same file
+        except ImportError as e:
+            raise LibraryMissing(f"the _native module is not built; run `python -m opengenie_amd.build` ({e})") from e
+        fn = _fns[name] = getattr(_native, name, None) or getattr(lib, name)
+    return fn
 
 
 def call(name: str, *args) -> None:
-    lib = load()
-    rc = getattr(lib, name)(*args)
+    rc = function(name)(*args)
     if rc != 0:
-        msg = lib.oga_last_error().decode() if rc < 0 else f"hipError {rc}"
+        msg = load().oga_last_error().decode() if rc < 0 else f"hipError {rc}"
         raise KernelError(f"{name} failed (rc={rc}): {msg}")

@@ -31,7 +31,7 @@ _FP8 = torch.float8_e4m3fn
 
 
 def _strides3(t: torch.Tensor):
-    return _lib.strides([t.stride(0), t.stride(1), t.stride(2)])
+    return _lib.strides(t.stride()[:3])
 
 
 def _kernel_ok(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
@@ -75,7 +75,7 @@ def _fp8_attention(q, k, v, q_descale, k_descale, v_descale, softmax_scale) -> t
     nk = k.shape[1]
     ds = [t.to(torch.float32).reshape(b, h).contiguous() for t in (q_descale, k_descale, v_descale)]
     out = torch.empty((b, nq, h, d), device=q.device, dtype=torch.bfloat16)
-    ws_bytes = int(_lib.load().oga_attention_fp8_workspace_bytes(b, nq, nk, h, d))
+    ws_bytes = _lib.function("oga_attention_fp8_workspace_bytes")(b, nq, nk, h, d)
     ws = torch.empty((ws_bytes,), device=q.device, dtype=torch.uint8)
     _hip("flash_attn_func_fp8")
     _lib.call("oga_attention_fp8_ws", q.data_ptr(), _strides3(q), k.data_ptr(), _strides3(k), v.data_ptr(),
@@ -146,10 +146,10 @@ def flash_attn_func(
     _hip("flash_attn_func")
     # Workspace for the key-split parts of a last partial round of blocks
     # (torch's caching allocator makes the per-call tensor cheap).
-    ws_bytes = int(_lib.load().oga_attention_workspace_bytes(b, nq, nk, h, d))
+    ws_bytes = _lib.function("oga_attention_workspace_bytes")(b, nq, nk, h, d)
     ws = torch.empty((ws_bytes // 4,), device=q.device, dtype=torch.float32) if ws_bytes else None
-    _lib.call("oga_attention_ws", q.data_ptr(), _strides3(q), k.data_ptr(), _strides3(k), v.data_ptr(), _strides3(v),
-              out.data_ptr(), _strides3(out), b, nq, nk, h, d, float(softmax_scale),
+    _lib.call("oga_attention_ws", q.data_ptr(), q.stride()[:3], k.data_ptr(), k.stride()[:3], v.data_ptr(),
+              v.stride()[:3], out.data_ptr(), out.stride()[:3], b, nq, nk, h, d, float(softmax_scale),
               ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q))
     return out
 
@@ -190,7 +190,7 @@ def attention_video_e4m3_out(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
     out = torch.empty((b, nq, heads * dim_head), device=q.device, dtype=_FP8)
     ov = out.view(b, nq, heads, dim_head)
     _hip("attention_video_e4m3_out")
-    ws_bytes = int(_lib.load().oga_attention_workspace_bytes(b, nq, nk, heads, dim_head))
+    ws_bytes = _lib.function("oga_attention_workspace_bytes")(b, nq, nk, heads, dim_head)
     ws = torch.empty((ws_bytes // 4,), device=q.device, dtype=torch.float32) if ws_bytes else None
     _lib.call("oga_attention_e4m3_out_ws", qv.data_ptr(), _strides3(qv), kv.data_ptr(), _strides3(kv), vv.data_ptr(),
               _strides3(vv), ov.data_ptr(), _strides3(ov), b, nq, nk, heads, dim_head, float(dim_head ** -0.5),

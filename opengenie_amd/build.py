@@ -1,9 +1,11 @@
-"""Builds libopengenie_amd.so (gfx950) from opengenie_amd/csrc with hipcc.
+"""Builds libopengenie_amd.so (gfx950) and its CPython binding _native from
+opengenie_amd/csrc with hipcc.
 
 Usage: python -m opengenie_amd.build [--jobs N]
 
 Every .hip source is compiled to an object in parallel, then linked into one
-shared library next to this file. Flags:
+shared library next to this file; pycall.cpp (host code) becomes the module
+_native beside it, linked to the library. Flags of the device sources:
   --offload-arch=gfx950         CDNA4 (MI355X) only
   -ffp-contract=off             no silent a*b+c fusion (bit-exact rounding)
   -target-feature -packed-fp32-ops
@@ -17,12 +19,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libopengenie_amd.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
+NATIVE_PATH = os.path.join(HERE, "_native" + sysconfig.get_config_var("EXT_SUFFIX"))
 BUILD_DIR = os.path.join(HERE, "_build")
 
 ARCH = "gfx950"
@@ -70,6 +74,14 @@ def build(jobs: int | None = None, verbose: bool = False) -> str:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
+    tmp = NATIVE_PATH + ".tmp"
+    cmd = [hipcc(), "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wl,--as-needed",
+           "-I" + sysconfig.get_paths()["include"], os.path.join(CSRC, "pycall.cpp"), "-o", tmp,
+           "-L" + HERE, "-lopengenie_amd", "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"_native failed:\n{' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, NATIVE_PATH)
     if verbose:
         print(f"built {LIB_PATH} from {len(srcs)} sources", file=sys.stderr)
     return LIB_PATH

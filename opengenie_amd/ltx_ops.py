@@ -70,6 +70,7 @@ __all__ = [
 
 _FP8 = torch.float8_e4m3fn
 _FP8_MAX = 448.0
+_DT_CODES = {torch.bfloat16: _lib.DT_BF16, torch.float16: _lib.DT_F16, torch.float32: _lib.DT_F32}
 
 # --------------------------------------------------------------------------
 # bookkeeping (mirrors the reference's module counters, :1992-2034)
@@ -149,11 +150,14 @@ def _xdt(t: torch.Tensor) -> int:
 
 def _any_dt(t: torch.Tensor) -> int:
     """dtype code of a bf16, fp16 or float32 tensor."""
-    return {torch.bfloat16: _lib.DT_BF16, torch.float16: _lib.DT_F16, torch.float32: _lib.DT_F32}[t.dtype]
+    return _DT_CODES[t.dtype]
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The raw handle of the current stream of t's device: what
+    torch.cuda.current_stream(t.device).cuda_stream holds, without the Stream
+    object made on each call."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -234,21 +238,20 @@ def _can_use_ada_from_table(x: torch.Tensor, scale_shift_table: torch.Tensor, ti
     most 65535 batches (one grid row per batch)."""
     if not x.is_cuda or not x.is_contiguous() or x.dtype != torch.bfloat16:
         return False
-    if x.ndim != 3 or x.shape[-1] not in (2048, 4096):
+    shape, table_shape, ts_shape = x.shape, scale_shift_table.shape, timestep.shape
+    if len(shape) != 3 or shape[2] not in (2048, 4096):
         return False
-    if not _aligned(x) or x.shape[0] > 65535:
+    if not _aligned(x) or shape[0] > 65535:
         return False
     if not scale_shift_table.is_cuda or scale_shift_table.dtype not in (torch.bfloat16, torch.float32):
         return False
-    if scale_shift_table.ndim != 2 or scale_shift_table.shape[-1] != x.shape[-1]:
+    if len(table_shape) != 2 or table_shape[1] != shape[2]:
         return False
-    if not timestep.is_cuda or timestep.dtype not in (torch.bfloat16, torch.float32) or timestep.ndim < 2:
+    if not timestep.is_cuda or timestep.dtype not in (torch.bfloat16, torch.float32) or len(ts_shape) < 2:
         return False
-    if timestep.shape[0] != x.shape[0] or timestep.shape[1] != x.shape[1]:
+    if ts_shape[0] != shape[0] or ts_shape[1] != shape[1]:
         return False
-    if timestep.numel() != x.shape[0] * x.shape[1] * scale_shift_table.shape[0] * x.shape[-1]:
-        return False
-    return True
+    return timestep.numel() == shape[0] * shape[1] * table_shape[0] * shape[2]
 
 
 def _can_use_fused_fp8_quantize(x: torch.Tensor, input_scale: torch.Tensor) -> bool:
@@ -430,9 +433,25 @@ def _ada_args(x: torch.Tensor, table: torch.Tensor, timestep: torch.Tensor, *ind
         if not -params <= i < params:
             raise IndexError(f"Ada index {i} out of range for a table with {params} rows")
     ts_view = timestep.reshape(x.shape[0], timestep.shape[1], params, x.shape[-1])
-    st = _lib.strides(ts_view.stride())
+    st = ts_view.stride()
     norm = [i % params for i in indices]
     return ts_view, st, norm
+
+
+def _ada_rows(x: torch.Tensor, table: torch.Tensor, timestep: torch.Tensor, *indices: int):
+    """_ada_args for callers that pass the view on as pointer and strides only:
+    a (B, N, P*C) timestep's (B, N, P, C) view starts where it starts and
+    splits its last stride, so no view is made."""
+    params, c = table.shape[0], x.shape[2]
+    if timestep.ndim != 3 or timestep.shape[2] != params * c:
+        return _ada_args(x, table, timestep, *indices)
+    norm = []
+    for i in indices:
+        if not -params <= i < params:
+            raise IndexError(f"Ada index {i} out of range for a table with {params} rows")
+        norm.append(i % params)
+    s0, s1, s2 = timestep.stride()
+    return timestep, (s0, s1, c * s2, s2), norm
 
 
 def _as_bnc(x: torch.Tensor) -> tuple[int, int, int]:
@@ -465,8 +484,8 @@ def fused_adazero(x: torch.Tensor, eps: float, scale: torch.Tensor, shift: torch
     b, n, c = _as_bnc(x)
     y = torch.empty_like(x)
     _hip("fused_adazero")
-    _lib.call("oga_adazero", _ptr(x), _ptr(y), b, n, c, _ptr(se), _dt(scale), _lib.strides(se.stride()), _ptr(he),
-              _dt(shift), _lib.strides(he.stride()), float(eps), _stream(x))
+    _lib.call("oga_adazero", x.data_ptr(), y.data_ptr(), b, n, c, _ptr(se), _dt(scale), se.stride(), _ptr(he),
+              _dt(shift), he.stride(), float(eps), _stream(x))
     return y
 
 
@@ -488,12 +507,12 @@ def fused_adazero_from_ada(
         )
         return fused_adazero(x, eps, scale, shift)
     _increment_ada_counter(counter)
-    ts_view, st, (si, ci) = _ada_args(x, scale_shift_table, timestep, shift_index, scale_index)
+    ts_view, st, (si, ci) = _ada_rows(x, scale_shift_table, timestep, shift_index, scale_index)
     y = torch.empty_like(x)
     _hip("fused_adazero_from_ada")
-    _lib.call("oga_adazero_from_ada", _ptr(x), _ptr(y), x.shape[0], x.shape[1], x.shape[2], _ptr(scale_shift_table),
-              _dt(scale_shift_table), scale_shift_table.stride(0), scale_shift_table.stride(1), _ptr(ts_view),
-              _dt(timestep), st, si, ci, float(eps), _stream(x))
+    _lib.call("oga_adazero_from_ada", x.data_ptr(), y.data_ptr(), *x.shape, scale_shift_table.data_ptr(),
+              _dt(scale_shift_table), *scale_shift_table.stride(), ts_view.data_ptr(), _dt(timestep), st, si, ci,
+              float(eps), _stream(x))
     return y
 
 
@@ -539,9 +558,9 @@ def fused_adazero_from_ada_fp8(
     _increment_ada_counter(counter)
     q = torch.empty(x.shape, device=x.device, dtype=_FP8)
     _hip("fused_adazero_from_ada_fp8")
-    _lib.call("oga_adazero_from_ada_fp8", _ptr(x), _ptr(q), x.shape[0], x.shape[1], x.shape[2],
-              _ptr(scale_shift_table), _dt(scale_shift_table), tab_s[0], tab_s[1], _ptr(ts_view), _dt(timestep), st,
-              si, ci, float(eps), _ptr(input_scale), int(input_scale.dim() == 0), _stream(x))
+    _lib.call("oga_adazero_from_ada_fp8", x.data_ptr(), q.data_ptr(), x.shape[0], x.shape[1], x.shape[2],
+              scale_shift_table.data_ptr(), _dt(scale_shift_table), tab_s[0], tab_s[1], ts_view.data_ptr(),
+              _dt(timestep), st, si, ci, float(eps), _ptr(input_scale), int(input_scale.dim() == 0), _stream(x))
     return q
 
 
@@ -562,12 +581,12 @@ def fused_adaln_affine_from_ada(
         )
         return x * (1 + scale) + shift
     _VIDEO_TEXT_ADALN_CALLS += 1
-    ts_view, st, (si, ci) = _ada_args(x, scale_shift_table, timestep, shift_index, scale_index)
+    ts_view, st, (si, ci) = _ada_rows(x, scale_shift_table, timestep, shift_index, scale_index)
     y = torch.empty_like(x)
     _hip("fused_adaln_affine_from_ada")
-    _lib.call("oga_adaln_affine_from_ada", _ptr(x), _ptr(y), x.shape[0], x.shape[1], x.shape[2],
-              _ptr(scale_shift_table), _dt(scale_shift_table), scale_shift_table.stride(0),
-              scale_shift_table.stride(1), _ptr(ts_view), _dt(timestep), st, si, ci, _stream(x))
+    _lib.call("oga_adaln_affine_from_ada", x.data_ptr(), y.data_ptr(), x.shape[0], x.shape[1], x.shape[2],
+              scale_shift_table.data_ptr(), _dt(scale_shift_table), scale_shift_table.stride(0),
+              scale_shift_table.stride(1), ts_view.data_ptr(), _dt(timestep), st, si, ci, _stream(x))
     return y
 
 
@@ -587,11 +606,11 @@ def fused_mul_from_ada(
         )
         return x * gate
     _VIDEO_TEXT_ADALN_CALLS += 1
-    ts_view, st, (gi,) = _ada_args(x, scale_shift_table, timestep, gate_index)
+    ts_view, st, (gi,) = _ada_rows(x, scale_shift_table, timestep, gate_index)
     y = torch.empty_like(x)
     _hip("fused_mul_from_ada")
-    _lib.call("oga_mul_from_ada", _ptr(x), _ptr(y), x.shape[0], x.shape[1], x.shape[2], _ptr(scale_shift_table),
-              _dt(scale_shift_table), scale_shift_table.stride(0), scale_shift_table.stride(1), _ptr(ts_view),
+    _lib.call("oga_mul_from_ada", x.data_ptr(), y.data_ptr(), *x.shape, scale_shift_table.data_ptr(),
+              _dt(scale_shift_table), scale_shift_table.stride(0), scale_shift_table.stride(1), ts_view.data_ptr(),
               _dt(timestep), st, gi, _stream(x))
     return y
 
@@ -628,12 +647,12 @@ def fused_residual_gate_from_ada(
         _increment_ada_counter("video")
     else:
         _increment_ada_counter("video_text")
-    ts_view, st, (gi,) = _ada_args(x, scale_shift_table, timestep, gate_index)
+    ts_view, st, (gi,) = _ada_rows(x, scale_shift_table, timestep, gate_index)
     out = torch.empty_like(x)
     _hip("fused_residual_gate_from_ada")
-    _lib.call("oga_residual_gate_from_ada", _ptr(x), _ptr(y), _ptr(out), x.shape[0], x.shape[1], x.shape[2],
-              _ptr(scale_shift_table), _dt(scale_shift_table), scale_shift_table.stride(0),
-              scale_shift_table.stride(1), _ptr(ts_view), _dt(timestep), st, gi, _stream(x))
+    _lib.call("oga_residual_gate_from_ada", x.data_ptr(), y.data_ptr(), out.data_ptr(), *x.shape,
+              scale_shift_table.data_ptr(), _dt(scale_shift_table), scale_shift_table.stride(0),
+              scale_shift_table.stride(1), ts_view.data_ptr(), _dt(timestep), st, gi, _stream(x))
     return out
 
 
@@ -666,14 +685,13 @@ def fused_residual_gate_bias_from_ada(
         _VIDEO_ADA_VALUES_CALLS += 1
     else:
         _VIDEO_TEXT_ADALN_CALLS += 1
-    ts_view, st, (gi,) = _ada_args(x, scale_shift_table, timestep, gate_index)
+    ts_view, st, (gi,) = _ada_rows(x, scale_shift_table, timestep, gate_index)
     bias_c = bias.contiguous()
     out = torch.empty_like(x)
     _hip("fused_residual_gate_bias_from_ada")
-    _lib.call("oga_residual_gate_bias_from_ada", _ptr(x), _ptr(y_no_bias), _ptr(bias_c), _dt(bias_c), _ptr(out),
-              x.shape[0], x.shape[1], x.shape[2], _ptr(scale_shift_table), _dt(scale_shift_table),
-              scale_shift_table.stride(0), scale_shift_table.stride(1), _ptr(ts_view), _dt(timestep), st, gi,
-              _stream(x))
+    _lib.call("oga_residual_gate_bias_from_ada", x.data_ptr(), y_no_bias.data_ptr(), bias_c.data_ptr(), _dt(bias_c),
+              out.data_ptr(), *x.shape, scale_shift_table.data_ptr(), _dt(scale_shift_table),
+              *scale_shift_table.stride(), ts_view.data_ptr(), _dt(timestep), st, gi, _stream(x))
     return out
 
 
@@ -745,10 +763,10 @@ def fused_residual_gate_adazero_from_ada(
     x_new = torch.empty_like(x)
     out = torch.empty(x.shape, device=x.device, dtype=_FP8) if input_scale is not None else torch.empty_like(x)
     _hip("fused_residual_gate_adazero_from_ada")
-    _lib.call("oga_residual_gate_adazero_from_ada", _ptr(x), _ptr(y), _ptr(bias_c),
-              _dt(bias_c) if bias_c is not None else 0, _ptr(x_new), _ptr(out), x.shape[0], x.shape[1], x.shape[2],
-              _ptr(scale_shift_table), _dt(scale_shift_table), tab_s[0], tab_s[1], _ptr(ts_view), _dt(timestep), st,
-              gi, si, ci, float(eps), _ptr(input_scale),
+    _lib.call("oga_residual_gate_adazero_from_ada", x.data_ptr(), y.data_ptr(), _ptr(bias_c),
+              _dt(bias_c) if bias_c is not None else 0, _ptr(x_new), out.data_ptr(), x.shape[0], x.shape[1], x.shape[2],
+              scale_shift_table.data_ptr(), _dt(scale_shift_table), tab_s[0], tab_s[1], ts_view.data_ptr(),
+              _dt(timestep), st, gi, si, ci, float(eps), _ptr(input_scale),
               int(input_scale.dim() == 0) if input_scale is not None else 0, _stream(x))
     return x_new, out
 
@@ -766,7 +784,7 @@ def fused_residual_gate_bf16(x: torch.Tensor, y: torch.Tensor, gate: torch.Tenso
     b, n, c = _as_bnc(x)
     out = torch.empty_like(x)
     _hip("fused_residual_gate_bf16")
-    _lib.call("oga_residual_gate_bf16", _ptr(x), _ptr(y), _ptr(ge), _lib.strides(ge.stride()), _ptr(out), b, n, c,
+    _lib.call("oga_residual_gate_bf16", x.data_ptr(), y.data_ptr(), ge.data_ptr(), ge.stride(), out.data_ptr(), b, n, c,
               _stream(x))
     return out
 
@@ -779,7 +797,7 @@ def fused_bias_add_bf16(x: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
     bias_c = bias.contiguous()
     out = torch.empty_like(x)
     _hip("fused_bias_add_bf16")
-    _lib.call("oga_bias_add_bf16", _ptr(x), _ptr(bias_c), _dt(bias_c), _ptr(out), x.numel() // x.shape[-1],
+    _lib.call("oga_bias_add_bf16", x.data_ptr(), _ptr(bias_c), _dt(bias_c), out.data_ptr(), x.numel() // x.shape[-1],
               x.shape[-1], _stream(x))
     return out
 
@@ -793,7 +811,7 @@ def fused_head_gate_mul_bf16(out: torch.Tensor, gates: torch.Tensor, heads: int,
     y = torch.empty_like(out)
     g2 = gates.reshape(-1, heads)
     _hip("fused_head_gate_mul_bf16")
-    _lib.call("oga_head_gate_mul_bf16", _ptr(out), _ptr(g2), g2.stride(0), g2.stride(1), _ptr(y),
+    _lib.call("oga_head_gate_mul_bf16", out.data_ptr(), _ptr(g2), g2.stride(0), g2.stride(1), y.data_ptr(),
               out.numel() // out.shape[-1], heads, dim_head, _stream(out))
     return y
 
@@ -810,7 +828,8 @@ def fused_fp8_quantize_e4m3(x: torch.Tensor, input_scale: torch.Tensor) -> torch
         return torch.clamp(x * input_scale.reciprocal(), fp8_min, fp8_max).to(_FP8)
     q = torch.empty_strided(x.shape, x.stride(), device=x.device, dtype=_FP8)
     _hip("fused_fp8_quantize_e4m3")
-    _lib.call("oga_fp8_quantize_e4m3", _ptr(x), _xdt(x), _ptr(input_scale), int(input_scale.dim() == 0), _ptr(q),
+    _lib.call("oga_fp8_quantize_e4m3", x.data_ptr(), _xdt(x), input_scale.data_ptr(), int(input_scale.dim() == 0),
+              q.data_ptr(),
               x.numel(), _stream(x))
     return q
 
@@ -829,7 +848,8 @@ def fused_gelu_tanh_fp8_quantize_e4m3(x: torch.Tensor, input_scale: torch.Tensor
         return torch.clamp(gelu * input_scale.reciprocal(), fp8_min, fp8_max).to(_FP8)
     q = torch.empty_strided(x.shape, x.stride(), device=x.device, dtype=_FP8)
     _hip("fused_gelu_tanh_fp8_quantize_e4m3")
-    _lib.call("oga_gelu_tanh_fp8_quantize_e4m3", _ptr(x), _xdt(x), _ptr(input_scale), int(input_scale.dim() == 0), _ptr(q),
+    _lib.call("oga_gelu_tanh_fp8_quantize_e4m3", x.data_ptr(), _xdt(x), input_scale.data_ptr(),
+              int(input_scale.dim() == 0), q.data_ptr(),
               x.numel(), _stream(x))
     return q
 
@@ -855,7 +875,8 @@ def fused_fp8_quantize_e4m3_per_head_4d(
     scale = torch.empty((batch, heads), device=x.device, dtype=torch.float32)
     q = torch.empty_strided(x.shape, x.stride(), device=x.device, dtype=_FP8)
     _hip("fused_fp8_quantize_e4m3_per_head_4d")
-    _lib.call("oga_fp8_quantize_per_head", _ptr(x), _xdt(x), _ptr(q), _ptr(scale), _ptr(workspace), batch, tokens, heads,
+    _lib.call("oga_fp8_quantize_per_head", x.data_ptr(), _xdt(x), q.data_ptr(), scale.data_ptr(),
+              workspace.data_ptr(), batch, tokens, heads,
               head_dim, _stream(x))
     return q, scale
 
@@ -870,7 +891,7 @@ def _rope_strides(cos: torch.Tensor, batch: int):
     st = list(cos.stride())
     if cos.shape[0] == 1:
         st[0] = 0
-    return cos, _lib.strides(st)
+    return cos, tuple(st)
 
 
 def fused_video_qk_rmsnorm_rope(
@@ -894,8 +915,9 @@ def fused_video_qk_rmsnorm_rope(
     q_out = torch.empty_like(q)
     k_out = torch.empty_like(k)
     _hip("fused_video_qk_rmsnorm_rope")
-    _lib.call("oga_video_qk_rmsnorm_rope", _ptr(q), _ptr(k), _ptr(qw), _ptr(kw), _dt(qw), _ptr(cos), _ptr(sin),
-              _dt(cos), cst, sst, _ptr(q_out), _ptr(k_out), q.shape[0], q.shape[1], q.shape[2], cos.shape[1],
+    _lib.call("oga_video_qk_rmsnorm_rope", q.data_ptr(), k.data_ptr(), qw.data_ptr(), kw.data_ptr(), _dt(qw),
+              cos.data_ptr(), sin.data_ptr(),
+              _dt(cos), cst, sst, q_out.data_ptr(), k_out.data_ptr(), q.shape[0], q.shape[1], q.shape[2], cos.shape[1],
               float(eps), _stream(q))
     return q_out, k_out
 
@@ -912,8 +934,8 @@ def fused_video_qk_rmsnorm_rope_separate(q, k, q_weight, k_weight, eps, cos, sin
     k_out = torch.empty_like(k)
     _hip("fused_video_qk_rmsnorm_rope_separate")
     for x, w, o in ((q, qw, q_out), (k, kw, k_out)):
-        _lib.call("oga_video_rmsnorm_rope", _ptr(x), _ptr(w), _dt(w), _ptr(cos), _ptr(sin), _dt(cos), cst, sst,
-                  _ptr(o), x.shape[0], x.shape[1], x.shape[2], cos.shape[1], float(eps), _stream(q))
+        _lib.call("oga_video_rmsnorm_rope", x.data_ptr(), w.data_ptr(), _dt(w), cos.data_ptr(), sin.data_ptr(), _dt(cos),
+                  cst, sst, o.data_ptr(), x.shape[0], x.shape[1], x.shape[2], cos.shape[1], float(eps), _stream(q))
     return q_out, k_out
 
 
@@ -931,8 +953,9 @@ def fused_video_qk_bias_rmsnorm_rope(q, k, q_bias, k_bias, q_weight, k_weight, e
     q_out = torch.empty_like(q)
     k_out = torch.empty_like(k)
     _hip("fused_video_qk_bias_rmsnorm_rope")
-    _lib.call("oga_video_qk_bias_rmsnorm_rope", _ptr(q), _ptr(k), _ptr(qb), _ptr(kb), _dt(qb), _ptr(qw), _ptr(kw),
-              _dt(qw), _ptr(cos), _ptr(sin), _dt(cos), cst, sst, _ptr(q_out), _ptr(k_out), q.shape[0], q.shape[1],
+    _lib.call("oga_video_qk_bias_rmsnorm_rope", q.data_ptr(), k.data_ptr(), _ptr(qb), _ptr(kb), _dt(qb), qw.data_ptr(),
+              kw.data_ptr(), _dt(qw), cos.data_ptr(), sin.data_ptr(), _dt(cos), cst, sst, q_out.data_ptr(),
+              k_out.data_ptr(), q.shape[0], q.shape[1],
               q.shape[2], cos.shape[1], float(eps), _stream(q))
     return q_out, k_out
 
@@ -960,7 +983,7 @@ def qk_rmsnorm(x: torch.Tensor, weight: torch.Tensor | None, eps: float) -> torc
         return torch.nn.functional.rms_norm(x, (cols,), weight=weight, eps=eps)
     out = torch.empty_like(x)
     _hip("qk_rmsnorm")
-    _lib.call("oga_rmsnorm", _ptr(x), _ptr(w), _dt(w) if w is not None else _lib.DT_BF16, _ptr(out),
+    _lib.call("oga_rmsnorm", x.data_ptr(), _ptr(w), _dt(w) if w is not None else _lib.DT_BF16, out.data_ptr(),
               x.numel() // cols, cols, float(eps), _stream(x))
     return out
 
@@ -978,8 +1001,9 @@ def fused_video_qkv_rmsnorm_rope_pack(q, k, v, q_weight, k_weight, eps, cos, sin
     sin, sst = _rope_strides(sin, batch)
     qkv = torch.empty((batch, tokens, 3, heads, cols // heads), device=q.device, dtype=q.dtype)
     _hip("fused_video_qkv_rmsnorm_rope_pack")
-    _lib.call("oga_video_qkv_rmsnorm_rope_pack", _ptr(q), _ptr(k), _ptr(v), _ptr(qw), _ptr(kw), _dt(qw), _ptr(cos),
-              _ptr(sin), _dt(cos), cst, sst, _ptr(qkv), batch, tokens, cols, heads, float(eps), _stream(q))
+    _lib.call("oga_video_qkv_rmsnorm_rope_pack", q.data_ptr(), k.data_ptr(), v.data_ptr(), qw.data_ptr(),
+              kw.data_ptr(), _dt(qw), cos.data_ptr(), sin.data_ptr(), _dt(cos), cst, sst, _ptr(qkv), batch,
+              tokens, cols, heads, float(eps), _stream(q))
     return qkv
 
 
@@ -994,19 +1018,21 @@ def _can_use_fp8_gemm(qflat: torch.Tensor, weight: torch.Tensor, scale_a, scale_
         return False
     if not (qflat.is_cuda and weight.is_cuda) or qflat.dtype != _FP8 or weight.dtype != _FP8:
         return False
-    if qflat.ndim != 2 or weight.ndim != 2 or qflat.shape[1] != weight.shape[1]:
+    q_shape, w_shape = qflat.shape, weight.shape
+    if len(q_shape) != 2 or len(w_shape) != 2 or q_shape[1] != w_shape[1]:
         return False
-    if qflat.stride(1) != 1 or weight.stride(1) != 1 or qflat.shape[1] % 128 != 0:
+    q_stride, w_stride = qflat.stride(), weight.stride()
+    if q_stride[1] != 1 or w_stride[1] != 1 or q_shape[1] % 128 != 0:
         return False
-    if qflat.stride(0) % 16 or weight.stride(0) % 16 or qflat.data_ptr() % 16 or weight.data_ptr() % 16:
+    if q_stride[0] % 16 or w_stride[0] % 16 or qflat.data_ptr() % 16 or weight.data_ptr() % 16:
         return False
-    if weight.shape[0] % 8:  # 16-byte output rows
+    if w_shape[0] % 8:  # 16-byte output rows
         return False
     for s in (scale_a, scale_b):
         if not isinstance(s, torch.Tensor) or s.numel() != 1 or not s.is_cuda or s.dtype != torch.float32:
             return False
     if bias is not None:
-        if not bias.is_cuda or bias.ndim != 1 or bias.shape[0] != weight.shape[0]:
+        if not bias.is_cuda or bias.ndim != 1 or bias.shape[0] != w_shape[0]:
             return False
         if bias.dtype not in (torch.bfloat16, torch.float32, torch.float16):
             return False
@@ -1045,11 +1071,11 @@ def fp8_scaled_mm(
     _hip("fp8_scaled_mm")
     # Split-K workspace for a last round of tiles that would not fill the
     # CUs (torch's caching allocator makes the per-call tensor cheap).
-    ws_bytes = int(_lib.load().oga_fp8_linear_workspace_bytes(m, n, k))
+    ws_bytes = _lib.function("oga_fp8_linear_workspace_bytes")(m, n, k)
     ws = torch.empty((ws_bytes // 4,), device=qinput.device, dtype=torch.float32) if ws_bytes else None
-    _lib.call("oga_fp8_linear_dt_ws", _ptr(qinput), qinput.stride(0), _ptr(weight), weight.stride(0),
-              _ptr(scale_a), _ptr(scale_b), _ptr(bias_c), _any_dt(bias_c) if bias_c is not None else 0, _ptr(out),
-              _xdt(out), out.stride(0), m, n, k, _ptr(ws), ws_bytes, _stream(qinput))
+    _lib.call("oga_fp8_linear_dt_ws", qinput.data_ptr(), qinput.stride(0), weight.data_ptr(), weight.stride(0),
+              scale_a.data_ptr(), scale_b.data_ptr(), _ptr(bias_c), _any_dt(bias_c) if bias_c is not None else 0,
+              out.data_ptr(), _xdt(out), n, m, n, k, _ptr(ws), ws_bytes, _stream(qinput))
     return out
 
 

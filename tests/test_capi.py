@@ -48,3 +48,30 @@ def test_abi_version_and_error_reporting():
     assert b"null" in lib.oga_last_error()
     rc = lib.oga_bias_add_bf16(None, None, 0, None, 1, 1, None)
     assert rc == -1
+
+
+@pytest.mark.skipif(not _lib.available(), reason="library not built")
+def test_native_module_binds_the_same_library():
+    """The compiled module's functions are the library's: arguments of every
+    kind (None, ints, a tuple and a ctypes array as int64_t arrays, a float)
+    reach the checks of the entry point, whose message the ctypes handle of
+    the same library reports; wrong counts and types raise."""
+    from opengenie_amd import _native
+
+    names = {n for n in dir(_native) if n.startswith("oga_")}
+    assert names and names <= set(_lib.SIGNATURES)
+    for st in ((1, 1, 1, 1), _lib.strides((1, 1, 1, 1))):
+        rc = _native.oga_adazero_from_ada(4096, 4096, 1, 1, 100, 4096, 0, 1, 1, 4096, 0, st, 0, 1, 1e-6, None)
+        assert rc < 0 and _lib.load().oga_last_error()
+    assert _lib.function("oga_bias_add_bf16")(None, None, 0, None, 1, 1, None) == -1
+    assert b"null" in _lib.load().oga_last_error()
+    with pytest.raises(TypeError):
+        _native.oga_bias_add_bf16(None)
+    with pytest.raises(TypeError):
+        _native.oga_bias_add_bf16(None, None, "0", None, 1, 1, None)
+    with pytest.raises(OverflowError):
+        _native.oga_bias_add_bf16(None, None, 1 << 40, None, 1, 1, None)
+    with pytest.raises(ValueError):
+        _native.oga_adazero_from_ada(4096, 4096, 1, 1, 4096, 4096, 0, 1, 1, 4096, 0, (1,) * 9, 0, 1, 1e-6, None)
+    with pytest.raises(_lib.KernelError):
+        _lib.call("oga_bias_add_bf16", None, None, 0, None, 1, 1, None)
