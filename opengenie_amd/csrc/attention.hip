@@ -659,15 +659,18 @@ __global__ __launch_bounds__(64 * kFewW) __attribute__((amdgpu_waves_per_eu(2, 2
   }
   char* const stage = (char*)smem + kFewStage + wv * kFewStageWave;
 
+  // Q^T fragments of a group's 32 queries (past nq the last query, never
+  // stored), read straight from HBM.
+  bf16x8 qf[8];
+  auto load_q = [&](int64_t grp) {
+    const int64_t qi = min(grp * 32 + ql, a.nq - 1);
+    const uint16_t* qrow = (const uint16_t*)a.q + b * a.q_sb + qi * a.q_sn + (int64_t)h * a.q_sh;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) qf[s] = __builtin_bit_cast(bf16x8, *(const uint4*)(qrow + 16 * s + 8 * hl));
+  };
+  load_q(min(g_begin + wv, ngroups - 1));
   for (int64_t grp = g_begin + wv; grp < g_end; grp += kFewW) {
     const int64_t q0 = grp * 32;
-    bf16x8 qf[8];
-    {
-      const int64_t qi = min(q0 + ql, a.nq - 1);
-      const uint16_t* qrow = (const uint16_t*)a.q + b * a.q_sb + qi * a.q_sn + (int64_t)h * a.q_sh;
-#pragma unroll
-      for (int s = 0; s < 8; ++s) qf[s] = __builtin_bit_cast(bf16x8, *(const uint4*)(qrow + 16 * s + 8 * hl));
-    }
     f32x16 o[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -703,6 +706,9 @@ __global__ __launch_bounds__(64 * kFewW) __attribute__((amdgpu_waves_per_eu(2, 2
       };
       sacc[0] = s_block(IC<0>{});
       sacc[1] = s_block(IC<1>{});
+      // The last S product has read the fragments: the wave's next group's
+      // go out here, under the softmax, P.V and output of this one.
+      if (ST + 1 == nsteps) load_q(min(grp + kFewW, ngroups - 1));
       auto read_v = [&](auto c_c, u32x2(&vr)[8]) {
         constexpr int OFF = ST * kParBytes + 4096 * decltype(c_c)::value;  // vaddr includes kVBuf
         vr[0] = lds_tr16<OFF>(vaddr[0][0]);
