@@ -671,12 +671,12 @@ __global__ __launch_bounds__(64 * kFewW) __attribute__((amdgpu_waves_per_eu(2, 2
   load_q(min(g_begin + wv, ngroups - 1));
   for (int64_t grp = g_begin + wv; grp < g_end; grp += kFewW) {
     const int64_t q0 = grp * 32;
+    // O^T, running max and sum: set by the first key step, which neither
+    // clears nor rescales them (the 128 instructions were a seventh of a
+    // group's at four steps).
     f32x16 o[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) o[i][e] = 0.0f;
-    float m_run = -INFINITY, l_run = 0.0f;
+    float m_run, l_run;
+    const f32x16 kZero16 = {};
 
     // One key step against resident pair ST (k_attention's s_phase,
     // softmax and pv_phase).
@@ -739,7 +739,9 @@ __global__ __launch_bounds__(64 * kFewW) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
         for (int e = (j == 0 ? 1 : 0); e < 16; ++e) mx = __builtin_fmaxf(mx, sacc[j][e]);
       const float ms = max_halves(mx) * a.scale_log2;
-      if (__any(ms > m_run + 8.0f)) {
+      if constexpr (ST == 0) {
+        m_run = ms;
+      } else if (__any(ms > m_run + 8.0f)) {
         const float m_new = __builtin_fmaxf(m_run, ms);
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
         l_run *= alpha;
@@ -762,7 +764,7 @@ __global__ __launch_bounds__(64 * kFewW) __attribute__((amdgpu_waves_per_eu(2, 2
           ps1 = (j == 0 && e == 0) ? p1 : ps1 + p1;
           pb[j][e >> 1] = pack2(p0, p1);
         }
-      l_run += ps0 + ps1;
+      l_run = ST == 0 ? ps0 + ps1 : l_run + (ps0 + ps1);
       auto pv = [&](auto c_c, u32x2(&cur)[8], u32x2(&nxt)[8]) {
         constexpr int C = decltype(c_c)::value;
         if constexpr (C + 1 < 4) {
@@ -779,7 +781,7 @@ __global__ __launch_bounds__(64 * kFewW) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
         for (int dblk = 0; dblk < 4; ++dblk) {
           const uint4 vu = {cur[2 * dblk][0], cur[2 * dblk][1], cur[2 * dblk + 1][0], cur[2 * dblk + 1][1]};
-          o[dblk] = mfma_bf16(__builtin_bit_cast(bf16x8, vu), pf, o[dblk]);
+          o[dblk] = mfma_bf16(__builtin_bit_cast(bf16x8, vu), pf, ST == 0 && C == 0 ? kZero16 : o[dblk]);
         }
       };
       pv(IC<0>{}, vr0, vr1);
