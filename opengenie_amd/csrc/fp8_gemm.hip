@@ -1199,7 +1199,7 @@ TileShape tile_shape(double slab_half, double slab_full, double round) {
 }
 const TileShape kTiles[] = {
     tile_shape<4, 4>(1.05, 1.37, 7.9), tile_shape<4, 3>(0.80, 1.03, 7.5), tile_shape<4, 2>(0.60, 0.74, 5.4),
-    tile_shape<2, 3>(0.54, 0.60, 4.1), tile_shape<2, 2>(0.41, 0.455, 2.8), tile_shape<2, 1>(0.35, 0.35, 2.3)};
+    tile_shape<2, 3>(0.54, 0.60, 4.1), tile_shape<2, 2>(0.425, 0.455, 2.8), tile_shape<2, 1>(0.35, 0.35, 2.3)};
 constexpr double kSplitUs = 13.7, kSplitChunkUs = 0.04;  // K-chunks and reduce: both launches, a chunk's partials
 
 // The tile with the shortest modelled time: whole rounds of the CUs, then the

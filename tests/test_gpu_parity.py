@@ -795,7 +795,7 @@ def test_fp8_linear_split_k_workspace_reuse(m, n, k):
     (1537, 4096, 896),                               # 128 x 256
     (2305, 4096, 640), (2400, 4224, 384),            # 192 x 256, and a last tile half past N
     (6144, 4096, 256),                               # two whole rounds of them
-    (64, 4096, 8192)])                               # K-chunks
+    (64, 4096, 16384)])                              # K-chunks of 256 x 256
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_fp8_linear_tiles(m, n, k, dtype):
     """The tiles of the persistent kernel at their edges (ragged rows and
