@@ -319,10 +319,12 @@ int oga_attention(const void* q, const int64_t q_strides[3], const void* k, cons
  * (16-byte aligned; 0 bytes and a null workspace run oga_attention). The
  * kernel runs one workgroup per 256-query block per CU at a time; the blocks
  * that would fill only part of a last round of the CUs (e.g. 1152 blocks on
- * 256 CUs at 9216 tokens x 32 heads) are cut into 2..8 parts over their keys,
- * whose float32 partial outputs, maxima and sums go to the workspace and are
+ * 256 CUs at 9216 tokens x 32 heads) are cut into 2..8 parts over their keys
+ * where that and the merge take less time than the whole blocks; the parts'
+ * float32 partial outputs, maxima and sums go to the workspace and are
  * merged by a second kernel on the same stream. Results agree with
- * oga_attention to float32 summation order. The size depends on the current
+ * oga_attention to float32 summation order. The size (a bound: a call that
+ * keeps its blocks whole leaves the workspace alone) depends on the current
  * device's CU count; a smaller workspace is an error.
  * Same interface as oga_attention (benchmarks/official_ltx23_benchmark.py:3294-3369).
  */

@@ -89,7 +89,7 @@ struct AttnArgs {
   float scale_log2;  // softmax scale * log2(e)
   // Workgroups 0 .. nfull-1 each own query block blockIdx.x (remapped) over
   // all keys. The blocks nfull .. end, which would fill only part of a last
-  // round of the CUs, are cut into ksplit parts over their key steps: later
+  // round of the CUs, may be cut into ksplit parts over their key steps: later
   // workgroup nfull + u owns part u % ksplit of block nfull + u / ksplit and
   // leaves its unnormalized O (part_o, [u][qpb][kAD] float32) and its
   // running max and sum (part_ml, [u][qpb][2]) for k_attention_combine.
