@@ -97,6 +97,13 @@ struct AttnArgs {
   int ksplit;
   float* part_o;
   float* part_ml;
+  // Blocks (of 256 queries for bf16, 384 for FP8, restart_nqb per head) from
+  // restart_from on begin a new running max where each of `restarts` parts of
+  // their key steps begins (attention_restarts); restart_magic is
+  // ceil(2^32 / restarts).
+  int64_t restart_from;
+  int restart_nqb;
+  uint32_t restarts, restart_magic;
   // FP8 kernel only: V rewritten as [B, H, D, vt_npad] (k_fp8_v_transpose)
   // and the [B, H] descales of q, k and v.
   const uint8_t* vt;
@@ -264,6 +271,29 @@ OGA_DEVICE float sum_halves(float v) {
 }
 
 
+// The key steps at which a block begins a new running max (AttnArgs): `next`
+// is the first one past the step last given to advance().
+struct Restarts {
+  uint32_t next = UINT32_MAX;  // (no step: keys stay below 2^32)
+  uint32_t p = 0;
+  // How far scores may pass the running max in step st before it moves: at a
+  // restart it always does.
+  OGA_DEVICE float lag(int64_t st, float usual) const { return (uint32_t)st == next ? -INFINITY : usual; }
+  // Part p begins at step floor(nsteps p / restarts): exact as the high word
+  // of the product with the magic while nsteps p < 2^29 (restarts <= 8).
+  OGA_DEVICE void advance(const AttnArgs& a, int64_t after) {
+    do {
+      ++p;
+      next = p < a.restarts ? __umulhi((uint32_t)((a.nk + kAK - 1) / kAK) * p, a.restart_magic) : UINT32_MAX;
+    } while (next <= (uint32_t)after);
+  }
+};
+// At a restart the running max becomes the max of that step's scores, at most
+// this far below the one before: seven restarts grow O and l by at most 2^28,
+// and a part whose scores all lie further down counts for less than 2^-4 of
+// its row.
+constexpr float kRestartDrop = 4.0f;
+
 // LDS: [K0 | V0 | K1 | V1 (| K2 | V2)], 16 KiB each; step st uses tile pair
 // st % BUFS, and the DMA of step st + BUFS - 1 goes out during step st.
 constexpr int kKBuf = 0, kVBuf = 16384, kParBytes = 32768;
@@ -321,6 +351,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   const int64_t nsteps_all = (a.nk + kAK - 1) / kAK;
   const int64_t st_begin = part < 0 ? 0 : nsteps_all * part / a.ksplit;
   const int64_t st_end = part < 0 ? nsteps_all : nsteps_all * (part + 1) / a.ksplit;
+  Restarts restarts;
+  if (BUFS == 3 && wg >= a.restart_from) restarts.advance(a, st_begin);
 
   f32x16 o[4];
 #pragma unroll
@@ -416,10 +448,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2))) 
   };
   // Online softmax of step st: keys past nk get score -inf; the running max
   // moves lazily (only when some query of the wave sees a score more than 8
-  // above it, always on the first step), so P = 2^(s scale_log2 - m_run) <=
-  // 256 and O, l are rescaled rarely. The float32 P feed l, their bf16
-  // roundings the P.V product (as FlashAttention does).
+  // above it, always on the first step and at a restart), so P =
+  // 2^(s scale_log2 - m_run) <= 256 and O, l are rescaled rarely. The float32
+  // P feed l, their bf16 roundings the P.V product (as FlashAttention does).
   auto softmax = [&](int64_t st, f32x16(&sacc)[2], uint32_t(&pb)[2][8]) {
+    const float lag = BUFS == 3 ? restarts.lag(st, 8.0f) : 8.0f;
     const int64_t rem64 = a.nk - st * kAK;
     if (rem64 < kAK) {
       const int remh = (int)rem64 - hl4;
@@ -436,8 +469,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       for (int e = (j == 0 ? 1 : 0); e < 16; ++e) mx = __builtin_fmaxf(mx, sacc[j][e]);
     // Base-2 scores s * scale_log2 (scale_log2 > 0, so the max commutes).
     const float ms = max_halves(mx) * a.scale_log2;
-    if (__any(ms > m_run + 8.0f)) {
-      const float m_new = __builtin_fmaxf(m_run, ms);
+    if (__any(ms > m_run + lag)) {
+      const bool restart = BUFS == 3 && lag < 0.0f;
+      const float m_new = __builtin_fmaxf(restart ? m_run - kRestartDrop : m_run, ms);
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);  // 0 on the first step (m_run = -inf)
       l_run *= alpha;
       m_run = m_new;
@@ -445,6 +479,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2))) 
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[i][e] *= alpha;
+      if (restart) restarts.advance(a, st);
     }
     const float nm = -m_run;
     float ps0, ps1;  // from the first terms (P >= 0 is never -0: 0 + x would be x)
@@ -866,8 +901,8 @@ constexpr float kF8Offset = 8.0f;  // P = 2^(s - m + kF8Offset): a row's largest
 // rescaled: at most 0.8, as 2^(8 + 0.8) = 445.7 stays below e4m3's largest
 // finite 448. The narrow form below lags by nothing: every score that sets a
 // new maximum then has P = 256, exact in e4m3, and the error against float64
-// attention falls from 0.0256 to 0.0250 at 4999 tokens (0.0251 -> 0.0246 at
-// 2304) for 3 % more time (324 against 334 us for the whole call).
+// attention falls from 0.0256 to 0.0250 at 4999 tokens for 3 % more time (324
+// against 334 us for the whole call).
 constexpr float kF8WideLag = 0.8f;
 static_assert(kF8Offset + kF8WideLag < 8.807f, "P must stay below 448 = 2^8.807");
 constexpr int kF8Pair = 2 * kF8Tile;
@@ -992,6 +1027,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(3, 3))) 
   const int64_t nsteps_all = (a.nk + kAK - 1) / kAK;
   const int64_t st_begin = part < 0 ? 0 : nsteps_all * part / a.ksplit;
   const int64_t st_end = part < 0 ? nsteps_all : nsteps_all * (part + 1) / a.ksplit;
+  Restarts restarts;
+  if (bh * a.restart_nqb + qb / (F8Cfg<kF8Wide>::kQ / kF8Q) >= a.restart_from) restarts.advance(a, st_begin);
 
   f32x16 o[4];
 #pragma unroll
@@ -1089,8 +1126,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(3, 3))) 
   // subnormals.) P goes in float32 into l and as e4m3 into the B operand,
   // byte 16j + e = P of accumulator e of block j; the common factor 2^8
   // cancels in O / l (and in the key-split merge, which weights O and l
-  // alike).
+  // alike). At a restart m moves to that step's max, down as well as up.
   auto softmax = [&](int64_t st, f32x16(&sacc)[2], i32x8& pf) {
+    const float lag = restarts.lag(st, kF8Lag);
     const int64_t rem64 = a.nk - st * kAK;
     if (rem64 < kAK) {
       const int remh = (int)rem64 - hl4;
@@ -1106,8 +1144,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(3, 3))) 
 #pragma unroll
       for (int e = (j == 0 ? 1 : 0); e < 16; ++e) mx = __builtin_fmaxf(mx, sacc[j][e]);
     const float ms = max_halves(mx) * sl2;
-    if (__any(ms > m_run + kF8Lag)) {
-      const float m_new = __builtin_fmaxf(m_run, ms);
+    if (__any(ms > m_run + lag)) {
+      const bool restart = lag < 0.0f;
+      const float m_new = __builtin_fmaxf(restart ? m_run - kRestartDrop : m_run, ms);
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
       l_run *= alpha;
       m_run = m_new;
@@ -1115,6 +1154,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(3, 3))) 
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[i][e] *= alpha;
+      if (restart) restarts.advance(a, st);
     }
     const float nm = kF8Offset - m_run;
     // (the sums start from their first term: P >= 0 is never -0, so 0 + x,
@@ -1443,6 +1483,33 @@ AttnPlan attention_plan(AttnKernel kern, int64_t wgs, int64_t nk, int64_t slots)
   if (p.ksplit > 1) { p.nfull = wgs - rem; p.units = rem * p.ksplit; }
   return p;
 }
+// A row in key parts has a running max of its own in each part: the largest P
+// of every part is then a rounded value near 1 (256 in e4m3), and those carry
+// the most of the error that rounding P makes. Blocks past the last whole
+// round of the bf16 kernel's or the wide FP8 form's workgroups, which a split
+// by rounds alone would cut in split_candidate parts, therefore begin a new
+// running max where such a part begins, whatever plan runs them, and err as
+// the parts do. The narrow FP8 form, whose max does not lag, is below that
+// without restarts where whole blocks are at least 3/5 of all or the parts
+// fewer than five. Error against float64 (2-norm, 32 heads) of blocks in
+// merged parts, of whole ones and of whole ones with restarts, and the time of
+// the call (FP8 without its quantizers; up to seven more rescalings and what
+// each new max brings):
+//   FP8  1025  0.0208 0.0232 0.0208   82  34  35 us
+//   FP8  2304  0.0232 0.0248 0.0232  117  77  80
+//   FP8  5500  0.0249 0.0259 0.0249  469 305 321
+//   bf16 1537  0.00226 0.00233 0.00226  144 51 52
+void attention_restarts(AttnArgs& a, AttnKernel kern, int64_t batch) {
+  const AttnKernel ref = kern == kFp8Narrow ? kFp8Wide : kern;
+  const int qpb = attn_cfg(ref).qpb;
+  const int64_t nqb = (a.nq + qpb - 1) / qpb, wgs = nqb * a.heads * batch;
+  const int64_t slots = attention_slots(ref), rem = slots > 0 ? wgs % slots : 0;
+  a.restart_nqb = (int)nqb;
+  a.restart_from = wgs - rem;
+  a.restarts = rem ? split_candidate(rem, a.nk, slots) : 1;
+  if (kern == kFp8Narrow && rem < wgs && (a.restarts < 5 || 5 * rem <= 2 * wgs)) a.restarts = 1;
+  a.restart_magic = (uint32_t)(((uint64_t(1) << 32) + a.restarts - 1) / a.restarts);
+}
 // The form of the FP8 kernel whose plan is the shorter one.
 AttnKernel fp8_kernel(int64_t batch, int64_t nq, int64_t nk, int64_t heads, AttnPlan* plan) {
   AttnKernel best = kFp8Wide;
@@ -1516,6 +1583,7 @@ int attention_run(const void* q, const int64_t q_strides[3], const void* k, cons
   if (nqb > INT32_MAX || wgs > UINT32_MAX / 8) return unsupported("too many query blocks");
   a.nqb = (int)nqb;
   a.qpb = cfg.qpb;
+  attention_restarts(a, kern, batch);
   AttnPlan plan{wgs, wgs, 0, 1, 0.0};
   if (workspace_bytes > 0) {
     const int64_t slots = attention_slots(kern);
@@ -1594,6 +1662,7 @@ int attention_fp8_run(const void* q, const int64_t q_strides[3], const void* k, 
     return unsupported("too many query blocks");
   AttnPlan plan{};
   const AttnKernel kern = fp8_kernel(batch, nq, nk, heads, &plan);
+  attention_restarts(a, kern, batch);
   const AttnCfg cfg = attn_cfg(kern);
   const int64_t nqb = (nq + cfg.qpb - 1) / cfg.qpb;
   const int64_t wgs = nqb * heads * batch;

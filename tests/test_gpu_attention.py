@@ -329,6 +329,106 @@ def test_fp8_attention_key_split():
     _check_fp8(out.float().cpu().numpy(), ref, _fp8_rounding_bound(qe, ke, ve), "fp8 key split")
 
 
+def _key_parts(n_blocks: int, cus: int, nk: int) -> tuple[int, int]:
+    """(first block, parts) of the blocks past the last whole round of the CUs
+    and the number of key parts that shortens that round the most (at least a
+    tenth of a round each time, at most 8; none up to 16 key steps)."""
+    rem, steps = n_blocks % cus, -(-nk // 64)
+    best, parts = 1.0, 1
+    for k in range(2, 9):
+        cost = -(-k * rem // cus) / k
+        if rem and steps > 16 and cost < best - 0.1:
+            best, parts = cost, k
+    return n_blocks - rem, parts
+
+
+def _parts_attention(s2, v, parts, offset, lag, rnd):
+    """Attention of one head, [N, NK] base-2 scores s2 and [NK, 128] values v
+    in float64, with P rounded by rnd as it enters the product: 64 keys at a
+    time, P = 2^(s2 - m + offset) against the running max m of 32 rows that
+    move together once one of them passes m + lag. Rows with parts > 1 take
+    their keys in that many parts with a running max of its own each."""
+    n, nk = s2.shape
+    steps = -(-nk // 64)
+    m = torch.full((n,), float("-inf"), device=s2.device, dtype=torch.float64)
+    o = torch.zeros((n, v.shape[1]), device=s2.device, dtype=torch.float64)
+    l = torch.zeros_like(m)
+    first = [torch.zeros_like(m, dtype=torch.bool) for _ in range(steps)]
+    for k in range(2, 9):
+        for p in range(1, k):
+            first[steps * p // k] |= parts == k
+    pad = -n % 32
+    for st in range(steps):
+        s, vs = s2[:, 64 * st:64 * st + 64], v[64 * st:64 * st + 64]
+        ms = s.amax(dim=1)
+        up = torch.nn.functional.pad(ms > m + lag, (0, pad)).view(-1, 32).any(dim=1).repeat_interleave(32)[:n]
+        new = torch.where(first[st], ms, torch.where(up, torch.maximum(m, ms), m))
+        alpha, m = torch.exp2(m - new), new
+        p = torch.exp2(s - m[:, None] + offset)
+        l = l * alpha + p.sum(dim=1)
+        o = o * alpha[:, None] + rnd(p) @ vs
+    return o / l[:, None]
+
+
+def _rel(x, ref) -> float:
+    return float((x.double() - ref).norm() / ref.norm())
+
+
+@pytest.mark.parametrize("b,n,h", [(1, 1025, 32), (1, 1537, 32), (2, 2004, 40), (1, 2304, 32), (1, 2500, 32),
+                                   (1, 4999, 32), (1, 5500, 32)])
+def test_fp8_attention_error_is_that_of_key_parts(b, n, h):
+    """FP8 self-attention where blocks of 384 queries past the last whole round
+    of the CUs could be cut in key parts: however they are run, the error
+    against float64 is at most what parts with a running max each (lagging by
+    up to 0.8) make of rounding P to e4m3. 1 % for the float32 scores, which
+    move a P across a rounding boundary now and then."""
+    from opengenie_amd.attention import flash_attn_func
+
+    q8, k8, v8 = (randn((b, n, h, 128), 940 + i + n).to(DEV).to(torch.float8_e4m3fn) for i in range(3))
+    one = torch.ones((b, h), device=DEV)
+    out = flash_attn_func(q8, k8, v8, q_descale=one, k_descale=one, v_descale=one)
+    _ran("flash_attn_func_fp8")
+    nqb = -(-n // 384)
+    start, k_parts = _key_parts(b * nqb * h, torch.cuda.get_device_properties(0).multi_processor_count, n)
+    errs, wants = [], []
+    for bi, head in ((0, 0), (b - 1, h // 2), (b - 1, h - 1)):  # (the first ones' blocks may be whole)
+        qd, kd, vd = (t[bi, :, head].double() for t in (q8, k8, v8))
+        s = (qd @ kd.t().contiguous()) * 128 ** -0.5
+        ref = torch.softmax(s, dim=-1) @ vd
+        block = (bi * h + head) * nqb + torch.arange(n, device=DEV) // 384
+        parts = torch.where(block >= start, k_parts, 1)
+        model = _parts_attention(s * np.log2(np.e), vd, parts, 8.0, 0.8,
+                                 lambda p: p.float().to(torch.float8_e4m3fn).double())
+        errs.append(_rel(out[bi, :, head], ref))
+        wants.append(_rel(model.to(torch.bfloat16), ref))
+    print(f"fp8 {b}x{n}x{h}: errors {errs}, key parts ({k_parts} from block {start}) {wants}")
+    assert np.mean(errs) <= 1.01 * np.mean(wants)
+
+
+@pytest.mark.parametrize("n", [1100, 1537, 3500])
+def test_attention_error_is_that_of_key_parts(n):
+    """The same for the bf16 kernel: 256 queries a block, P rounded to bf16
+    against a running max that lags by up to 8."""
+    from opengenie_amd.attention import flash_attn_func
+
+    h = 32
+    q, k, v = (randn((1, n, h, 128), 945 + i + n).to(DEV) for i in range(3))
+    out = flash_attn_func(q, k, v)
+    _ran("flash_attn_func")
+    nqb = -(-n // 256)
+    start, k_parts = _key_parts(nqb * h, torch.cuda.get_device_properties(0).multi_processor_count, n)
+    for head in (19, 31):
+        qd, kd, vd = (t[0, :, head].double() for t in (q, k, v))
+        s = (qd @ kd.t().contiguous()) * 128 ** -0.5
+        ref = torch.softmax(s, dim=-1) @ vd
+        block = head * nqb + torch.arange(n, device=DEV) // 256
+        parts = torch.where(block >= start, k_parts, 1)
+        model = _parts_attention(s * np.log2(np.e), vd, parts, 0.0, 8.0, lambda p: p.to(torch.bfloat16).double())
+        err, want = _rel(out[0, :, head], ref), _rel(model.to(torch.bfloat16), ref)
+        print(f"bf16 {n} head {head}: error {err:.6f}, key parts ({k_parts} from block {start}) {want:.6f}")
+        assert err <= 1.01 * want, (n, head, err, want)
+
+
 def test_fp8_attention_strided_views():
     """q, k, v as strided [B, N, H, D] views of one packed e4m3 buffer."""
     from opengenie_amd.attention import flash_attn_func
