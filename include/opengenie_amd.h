@@ -323,9 +323,9 @@ int oga_attention(const void* q, const int64_t q_strides[3], const void* k, cons
  * where that and the merge take less time than the whole blocks; the parts'
  * float32 partial outputs, maxima and sums go to the workspace and are
  * merged by a second kernel on the same stream. Results agree with
- * oga_attention to float32 summation order. The size (a bound: a call that
- * keeps its blocks whole leaves the workspace alone) depends on the current
- * device's CU count; a smaller workspace is an error.
+ * oga_attention to float32 summation order. The size, 0 for a call that keeps
+ * its blocks whole, depends on the current device's CU count; a smaller
+ * workspace is an error.
  * Same interface as oga_attention (benchmarks/official_ltx23_benchmark.py:3294-3369).
  */
 int64_t oga_attention_workspace_bytes(int64_t batch, int64_t nq, int64_t nk, int64_t heads, int64_t head_dim);
@@ -333,6 +333,16 @@ int oga_attention_ws(const void* q, const int64_t q_strides[3], const void* k, c
                      const void* v, const int64_t v_strides[3], void* o, const int64_t o_strides[3], int64_t batch,
                      int64_t nq, int64_t nk, int64_t heads, int64_t head_dim, float softmax_scale, void* workspace,
                      int64_t workspace_bytes, void* stream);
+
+/*
+ * The schedule of such a call (fp8 0) or of oga_attention_fp8_ws (fp8 not 0),
+ * without running it: plan[0] queries per block, plan[1] blocks, plan[2]
+ * blocks run whole and plan[3] the key parts of each other one (1: none).
+ * cus 0 asks the current device, a positive number is a gfx950 of that many
+ * CUs. (Up to 256 bf16 keys a kernel of its own runs, which has no plan.) No
+ * counterpart in the reference.
+ */
+int oga_attention_plan(int fp8, int64_t batch, int64_t nq, int64_t nk, int64_t heads, int64_t cus, int64_t plan[4]);
 
 /*
  * oga_attention_ws whose output goes straight into the input quantizer of

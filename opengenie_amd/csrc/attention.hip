@@ -1386,13 +1386,14 @@ enum AttnKernel { kBf16Long = 0, kBf16Short = 1, kFp8Wide = 2, kFp8Narrow = 3 };
 struct AttnCfg {
   const void* fn;
   int threads, qpb;
+  int per_cu;  // workgroups a CU of the gfx950 holds
 };
 AttnCfg attn_cfg(AttnKernel k) {
   switch (k) {
-    case kBf16Short: return {(const void*)k_attention<kAWShort, kABufsShort>, 64 * kAWShort, 32 * kAWShort};
-    case kFp8Wide: return {(const void*)k_attention_fp8<kF8Wide>, 64 * kF8Wide, F8Cfg<kF8Wide>::kQ};
-    case kFp8Narrow: return {(const void*)k_attention_fp8<kF8Narrow>, 64 * kF8Narrow, F8Cfg<kF8Narrow>::kQ};
-    default: return {(const void*)k_attention<kAW, kABufs>, 64 * kAW, kAQ};
+    case kBf16Short: return {(const void*)k_attention<kAWShort, kABufsShort>, 64 * kAWShort, 32 * kAWShort, 2};
+    case kFp8Wide: return {(const void*)k_attention_fp8<kF8Wide>, 64 * kF8Wide, F8Cfg<kF8Wide>::kQ, 1};
+    case kFp8Narrow: return {(const void*)k_attention_fp8<kF8Narrow>, 64 * kF8Narrow, F8Cfg<kF8Narrow>::kQ, 3};
+    default: return {(const void*)k_attention<kAW, kABufs>, 64 * kAW, kAQ, 1};
   }
 }
 AttnKernel bf16_kernel(int64_t nk) { return (nk + kAK - 1) / kAK <= kShortSteps ? kBf16Short : kBf16Long; }
@@ -1400,7 +1401,9 @@ AttnKernel bf16_kernel(int64_t nk) { return (nk + kAK - 1) / kAK <= kShortSteps 
 // Workgroups of an attention kernel resident at once on the current device
 // (CUs x workgroups per CU), cached per device (relaxed atomics: threads
 // filling an entry at once store the same value); 0 if the runtime cannot say.
-int64_t attention_slots(AttnKernel kern) {
+// cus_of > 0: of a gfx950 with that many CUs instead, no device asked.
+int64_t attention_slots(AttnKernel kern, int64_t cus_of = 0) {
+  if (cus_of > 0) return cus_of * attn_cfg(kern).per_cu;
   static std::atomic<int64_t> cache[4][64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
@@ -1428,8 +1431,7 @@ struct AttnPlan {
 // stores, which every part repeats, and the merge adds a launch (at 256 keys
 // the split ran 75.7 against 66.9 us unsplit). split_candidate is the k with
 // the shortest last round alone (ceil(k rem / slots) rounds of 1/k of a
-// block's time, shorter by at least a tenth of a round); it sizes the
-// workspace.
+// block's time, shorter by at least a tenth of a round).
 int split_candidate(int64_t rem, int64_t nk, int64_t slots) {
   const int64_t nsteps = (nk + kAK - 1) / kAK;
   int ksplit = 1;
@@ -1511,22 +1513,14 @@ void attention_restarts(AttnArgs& a, AttnKernel kern, int64_t batch) {
   a.restart_magic = (uint32_t)(((uint64_t(1) << 32) + a.restarts - 1) / a.restarts);
 }
 // The form of the FP8 kernel whose plan is the shorter one.
-AttnKernel fp8_kernel(int64_t batch, int64_t nq, int64_t nk, int64_t heads, AttnPlan* plan) {
+AttnKernel fp8_kernel(int64_t batch, int64_t nq, int64_t nk, int64_t heads, AttnPlan* plan, int64_t cus_of = 0) {
   AttnKernel best = kFp8Wide;
   for (AttnKernel kern : {kFp8Wide, kFp8Narrow}) {
     const int qpb = attn_cfg(kern).qpb;
-    const AttnPlan p = attention_plan(kern, (nq + qpb - 1) / qpb * heads * batch, nk, attention_slots(kern));
+    const AttnPlan p = attention_plan(kern, (nq + qpb - 1) / qpb * heads * batch, nk, attention_slots(kern, cus_of));
     if (kern == kFp8Wide || p.us < plan->us) { *plan = p; best = kern; }
   }
   return best;
-}
-// Bytes of partials the largest split of this shape could take: an upper
-// bound of what attention_plan uses, which keeps blocks whole where the
-// merge would cost more than it gains.
-int64_t attention_ws_bound(int64_t wgs, int64_t nk, int64_t slots, int qpb) {
-  const int64_t rem = slots > 0 ? wgs % slots : 0;
-  const int k = rem ? split_candidate(rem, nk, slots) : 1;
-  return k > 1 ? rem * k * qpb * (kAD + 2) * (int64_t)sizeof(float) : 0;
 }
 int64_t attention_ws_bytes(const AttnPlan& p, int qpb) { return p.units * qpb * (kAD + 2) * (int64_t)sizeof(float); }
 
@@ -1586,10 +1580,9 @@ int attention_run(const void* q, const int64_t q_strides[3], const void* k, cons
   attention_restarts(a, kern, batch);
   AttnPlan plan{wgs, wgs, 0, 1, 0.0};
   if (workspace_bytes > 0) {
-    const int64_t slots = attention_slots(kern);
-    if (attention_ws_bound(wgs, nk, slots, cfg.qpb) > workspace_bytes)
+    plan = attention_plan(kern, wgs, nk, attention_slots(kern));
+    if (attention_ws_bytes(plan, cfg.qpb) > workspace_bytes)
       return fail("workspace smaller than oga_attention_workspace_bytes");
-    plan = attention_plan(kern, wgs, nk, slots);
   }
   a.nfull = plan.nfull;
   a.ksplit = plan.ksplit;
@@ -1708,7 +1701,7 @@ extern "C" int64_t oga_attention_workspace_bytes(int64_t batch, int64_t nq, int6
   const int qpb = attn_cfg(kern).qpb;
   const int64_t nqb = (nq + qpb - 1) / qpb;
   if (nqb > INT32_MAX || heads > INT32_MAX || nqb * heads > (int64_t)(UINT32_MAX / 8) / batch) return 0;
-  return attention_ws_bound(nqb * heads * batch, nk, attention_slots(kern), qpb);
+  return attention_ws_bytes(attention_plan(kern, nqb * heads * batch, nk, attention_slots(kern)), qpb);
 }
 
 extern "C" int oga_attention_ws(const void* q, const int64_t q_strides[3], const void* k, const int64_t k_strides[3],
@@ -1728,6 +1721,27 @@ extern "C" int oga_attention_e4m3_out_ws(const void* q, const int64_t q_strides[
   if (!out_scale) return fail("null output scale");
   return attention_run(q, q_strides, k, k_strides, v, v_strides, o8, o_strides, batch, nq, nk, heads, head_dim,
                        softmax_scale, workspace, workspace_bytes, stream, out_scale, scale_zero_dim);
+}
+
+extern "C" int oga_attention_plan(int fp8, int64_t batch, int64_t nq, int64_t nk, int64_t heads, int64_t cus,
+                                  int64_t plan[4]) {
+  if (!plan) return fail("null pointer");
+  if (batch <= 0 || nq <= 0 || nk <= 0 || heads <= 0 || cus < 0) return fail("bad shape");
+  if (heads > INT32_MAX / batch || (nq + 127) / 128 > (int64_t)(UINT32_MAX / 8) / (heads * batch))
+    return unsupported("too many query blocks");
+  AttnPlan p{};
+  AttnKernel kern = bf16_kernel(nk);
+  if (fp8) {
+    kern = fp8_kernel(batch, nq, nk, heads, &p, cus);
+  } else {
+    const int qpb = attn_cfg(kern).qpb;
+    p = attention_plan(kern, (nq + qpb - 1) / qpb * heads * batch, nk, attention_slots(kern, cus));
+  }
+  plan[0] = attn_cfg(kern).qpb;
+  plan[1] = p.wgs;
+  plan[2] = p.nfull;
+  plan[3] = p.ksplit;
+  return OGA_OK;
 }
 
 extern "C" int64_t oga_attention_fp8_workspace_bytes(int64_t batch, int64_t nq, int64_t nk, int64_t heads,

@@ -75,3 +75,32 @@ def test_native_module_binds_the_same_library():
         _native.oga_adazero_from_ada(4096, 4096, 1, 1, 4096, 4096, 0, 1, 1, 4096, 0, (1,) * 9, 0, 1, 1e-6, None)
     with pytest.raises(_lib.KernelError):
         _lib.call("oga_bias_add_bf16", None, None, 0, None, 1, 1, None)
+
+
+def _attention_plan(fp8, batch, nq, nk, heads, cus=256):
+    plan = (ctypes.c_int64 * 4)()
+    assert _lib.load().oga_attention_plan(fp8, batch, nq, nk, heads, cus, plan) == 0
+    return tuple(plan)
+
+
+@pytest.mark.skipif(not _lib.available(), reason="library not built")
+def test_attention_plans():
+    """Schedules on 256 CUs: the blocks of a plan cover the queries, whole ones
+    fill rounds of the resident workgroups, parts are two to eight and no
+    shorter than a key step, and none up to 16 key steps; the forms and splits
+    of a few shapes as their comments in the kernels' source describe them."""
+    for fp8, n in [(f, n) for f in (0, 1) for n in (1, 63, 512, 1024, 1025, 1537, 2304, 3500, 4999, 9216, 14080)]:
+        for batch, heads in ((1, 32), (1, 1), (2, 24), (3, 40)):
+            qpb, blocks, full, parts = _attention_plan(fp8, batch, n, n, heads)
+            slots = {(0, 256): 256, (0, 128): 512, (1, 384): 256, (1, 128): 768}[fp8, qpb]
+            assert blocks == batch * heads * -(-n // qpb) and 1 <= parts <= 8
+            assert full == blocks if parts == 1 else full == blocks // slots * slots < blocks
+            assert parts == 1 or n > 1024
+    assert _attention_plan(0, 1, 1537, 1537, 32) == (256, 224, 224, 1)
+    assert _attention_plan(0, 1, 9216, 9216, 32) == (256, 1152, 1024, 2)
+    assert _attention_plan(1, 1, 4999, 4999, 32) == (128, 1280, 1280, 1)
+    assert _attention_plan(1, 1, 4352, 4352, 32) == (384, 384, 256, 2)
+    assert _attention_plan(1, 1, 9216, 9216, 32) == (384, 768, 768, 1)
+    lib = _lib.load()
+    assert lib.oga_attention_plan(0, 1, 1, 1, 1, 256, None) < 0
+    assert lib.oga_attention_plan(0, 1, 0, 1, 1, 256, (ctypes.c_int64 * 4)()) < 0

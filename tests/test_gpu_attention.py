@@ -78,19 +78,35 @@ def test_attention_matches_oracle(b, nq, nk, h):
     _check(out, _ref(q, k, v), f"attn b{b} nq{nq} nk{nk} h{h}")
 
 
-@pytest.mark.parametrize("b,nq,nk,h", [(1, 128, 1100, 1), (1, 2048, 1500, 20)])
+def _plan(fp8: bool, b: int, nq: int, nk: int, h: int) -> tuple[int, int, int, int]:
+    """(queries per block, blocks, blocks run whole, key parts of the others)
+    of an attention call on this device."""
+    import ctypes
+
+    from opengenie_amd import _lib
+
+    plan = (ctypes.c_int64 * 4)()
+    assert _lib.load().oga_attention_plan(int(fp8), b, nq, nk, h, 0, plan) == 0
+    return tuple(plan)
+
+
+@pytest.mark.parametrize("b,nq,nk,h", [(1, 128, 1100, 1), (1, 2304, 1500, 29)])
 def test_attention_key_split_and_whole_agree(b, nq, nk, h):
     """flash_attn_func cuts a last partial round of query blocks into key
     parts merged by a second kernel (oga_attention_ws; only beyond 16 key
-    steps); oga_attention runs every block over all keys. Both meet the
-    oracle bar, and they differ only in float32 summation order."""
+    steps) where that is modelled shorter: one block in eight parts, and five
+    blocks past a whole round of 256 (asserted from the plan). oga_attention
+    runs every block over all keys. Both meet the oracle bar, and they differ
+    only in float32 summation order."""
     from opengenie_amd import _lib
     from opengenie_amd.attention import _strides3, flash_attn_func
 
     q = randn((b, nq, h, 128), 800 + nq).to(DEV)
     k = randn((b, nk, h, 128), 801 + nk).to(DEV)
     v = randn((b, nk, h, 128), 802 + nk).to(DEV)
-    assert _lib.load().oga_attention_workspace_bytes(b, nq, nk, h, 128) > 0  # the split path runs
+    qpb, blocks, full, parts = _plan(False, b, nq, nk, h)
+    assert parts > 1 and full < blocks and (full > 0) == (blocks > 256)
+    assert _lib.load().oga_attention_workspace_bytes(b, nq, nk, h, 128) == (blocks - full) * parts * qpb * 130 * 4
     split = flash_attn_func(q, k, v)
     whole = torch.empty_like(q)
     _lib.call("oga_attention", q.data_ptr(), _strides3(q), k.data_ptr(), _strides3(k), v.data_ptr(), _strides3(v),
@@ -102,6 +118,15 @@ def test_attention_key_split_and_whole_agree(b, nq, nk, h):
     _check(whole, ref, f"attn whole b{b} nq{nq} nk{nk} h{h}")
     diff = (split.float() - whole.float()).abs()
     assert float(diff.max()) <= 2 ** -7 * float(whole.float().abs().max()), float(diff.max())
+
+
+def test_attention_workspace_is_what_the_plan_uses():
+    """Calls whose blocks all run whole take no workspace: 224 blocks of 1537
+    tokens x 32 heads, which a split by rounds alone would cut in eight."""
+    from opengenie_amd import _lib
+
+    assert _plan(False, 1, 1537, 1537, 32) == (256, 224, 224, 1)
+    assert _lib.load().oga_attention_workspace_bytes(1, 1537, 1537, 32, 128) == 0
 
 
 def test_attention_workspace_contract():
@@ -277,7 +302,7 @@ def test_fp8_attention_kernel(b, nq, nk, h):
 
 @pytest.mark.parametrize("b,nq,nk,h", [(1, 1, 1, 8), (1, 127, 63, 8), (2, 128, 64, 8), (1, 129, 65, 8), (1, 385, 193, 8),
                                        (1, 256, 2113, 8),   # 16 workgroups, 34 key steps: key parts and their merge
-                                       (1, 4480, 300, 8)])  # more workgroups than one per CU
+                                       (1, 4480, 300, 8)])  # more workgroups than CUs: two on some
 def test_fp8_attention_narrow_form_edges(b, nq, nk, h):
     """The FP8 kernel's 4-wave form at the edges of its 128-query blocks and
     64-key steps, with a partial last step, with its key-split parts and with
@@ -286,6 +311,9 @@ def test_fp8_attention_narrow_form_edges(b, nq, nk, h):
     from opengenie_amd.attention import flash_attn_func
     from opengenie_amd.ltx_ops import fused_fp8_quantize_e4m3_per_head_4d
 
+    qpb, blocks, full, parts = _plan(True, b, nq, nk, h)
+    assert qpb == 128 and blocks == b * h * -(-nq // 128)
+    assert (parts > 1 and full == 0) if nk == 2113 else full == blocks
     q, k, v = (randn((b, n, h, 128), 970 + i + n).to(DEV) for i, n in enumerate((nq, nk, nk)))
     (q8, qs), (k8, ks), (v8, vs) = (fused_fp8_quantize_e4m3_per_head_4d(t) for t in (q, k, v))
     out = flash_attn_func(q8, k8, v8, q_descale=qs, k_descale=ks, v_descale=vs)
@@ -300,33 +328,38 @@ def test_fp8_attention_narrow_form_edges(b, nq, nk, h):
         assert (np.abs(got - ref) <= (1 + 2.0 ** -6) * bound + 2.0 ** -8 * np.abs(ref) + 1e-6).all()
 
 
-def test_fp8_attention_key_split():
-    """17 query blocks x 16 heads = 272 workgroups of the FP8 kernel: on a
-    256-CU device the 16 past the whole round run as key parts merged by the
-    combine kernel (asserted from the workspace query, which then exceeds the
-    V rewrite; 1100 keys, more than the 16 steps below which no split is
-    made). Against float64 attention with the e4m3 bars."""
+@pytest.mark.parametrize("nq,nk,h,form,heads", [(6528, 1100, 16, 128, (0, 15)), (4352, 4352, 32, 384, (0, 20, 21, 31))])
+def test_fp8_attention_key_split(nq, nk, h, form, heads):
+    """Both forms of the FP8 kernel with whole rounds of workgroups and key
+    parts after them, merged by the combine kernel, against float64 attention
+    with the e4m3 bars. On 256 CUs the 4-wave form runs 768 of 816 blocks of
+    128 queries whole (the rest are head 15's from its fourth block on), the
+    12-wave form 256 of 384 blocks of 384 (the rest from head 21's fifth)."""
     from opengenie_amd import _lib
     from opengenie_amd.attention import flash_attn_func
     from opengenie_amd.ltx_ops import fused_fp8_quantize_e4m3_per_head_4d
 
-    b, nq, nk, h = 1, 17 * 384, 1100, 16
-    lib = _lib.load()
-    vt_bytes = b * h * 128 * ((nk + 63) // 64 * 64)
-    if int(lib.oga_attention_fp8_workspace_bytes(b, nq, nk, h, 128)) <= vt_bytes:
-        pytest.skip("this device runs the 272 workgroups without a key split")
-    q = randn((b, nq, h, 128), 940).to(DEV)
-    k = randn((b, nk, h, 128), 941).to(DEV)
-    v = randn((b, nk, h, 128), 942).to(DEV)
+    qpb, blocks, full, parts = _plan(True, 1, nq, nk, h)
+    assert qpb == form and 0 < full < blocks and parts > 1
+    vt_bytes = h * 128 * ((nk + 63) // 64 * 64)
+    assert _lib.load().oga_attention_fp8_workspace_bytes(1, nq, nk, h, 128) == \
+        vt_bytes + (blocks - full) * parts * qpb * 130 * 4
+    q = randn((1, nq, h, 128), 940).to(DEV)
+    k = randn((1, nk, h, 128), 941).to(DEV)
+    v = randn((1, nk, h, 128), 942).to(DEV)
     q8, qs = fused_fp8_quantize_e4m3_per_head_4d(q)
     k8, ks = fused_fp8_quantize_e4m3_per_head_4d(k)
     v8, vs = fused_fp8_quantize_e4m3_per_head_4d(v)
     out = flash_attn_func(q8, k8, v8, q_descale=qs, k_descale=ks, v_descale=vs)
     torch.cuda.synchronize()
     _ran("flash_attn_func_fp8")
-    qe, ke, ve = (_fp8_exact(t, s) for t, s in ((q8, qs), (k8, ks), (v8, vs)))
+    rows = np.unique(np.concatenate([np.arange(0, nq, 13), [nq - 1]]))
+    hs = list(heads)
+    qe, ke, ve = (_fp8_exact(t[:, :, hs], s[:, hs]) for t, s in ((q8, qs), (k8, ks), (v8, vs)))
+    qe = qe[:, rows]
     ref = O.attention(*[np.ascontiguousarray(x.transpose(0, 2, 1, 3)) for x in (qe, ke, ve)]).transpose(0, 2, 1, 3)
-    _check_fp8(out.float().cpu().numpy(), ref, _fp8_rounding_bound(qe, ke, ve), "fp8 key split")
+    got = out[:, :, hs].float().cpu().numpy()[:, rows]
+    _check_fp8(got, ref, _fp8_rounding_bound(qe, ke, ve), f"fp8 key split, blocks of {form}")
 
 
 def _key_parts(n_blocks: int, cus: int, nk: int) -> tuple[int, int]:
@@ -475,7 +508,7 @@ def test_fp8_attention_config_shape_against_bf16():
     print("fp8 vs bf16 at 1x9216x32x128:", stats)
     assert stats["rms"] < 0.12 * float(ref16.square().mean().sqrt()), stats
     heads = [0, 7, 19, 31]
-    rows = np.arange(0, n, 97)  # 96 query rows, both split and whole query blocks
+    rows = np.arange(0, n, 97)  # 96 query rows
     qe = _fp8_exact(q8, qs)[:, rows][:, :, heads]
     ke = _fp8_exact(k8, ks)[:, :, heads]
     ve = _fp8_exact(v8, vs)[:, :, heads]
@@ -495,8 +528,7 @@ def test_attention_config_shape():
     from opengenie_amd.attention import flash_attn_func
 
     n, h = 9216, 32
-    lib = _lib.load()
-    assert int(lib.oga_attention_workspace_bytes(1, n, n, h, 128)) > 0  # the key split is planned
+    assert _plan(False, 1, n, n, h) == (256, 1152, 1024, 2)  # (256 CUs) the key split is planned
     q, k, v = (randn((1, n, h, 128), 960 + i) for i in range(3))
     out = flash_attn_func(q.to(DEV), k.to(DEV), v.to(DEV))
     torch.cuda.synchronize()
