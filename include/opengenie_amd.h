@@ -256,11 +256,21 @@ int oga_fp8_linear(const void* a, int64_t lda, const void* w, int64_t ldw, const
  * the tiles of that round may be cut into K-chunks whose float32 partial
  * sums go to the workspace and are added in chunk order (deterministic);
  * the chunk count weighs the chunks' time against the partials' traffic,
- * and the size is 0 when no cut of 256 x 256 tiles pays. The call leaves the
- * workspace alone where a smaller tile, whole, is faster still. A null or
- * smaller workspace (and a size of 0) runs oga_fp8_linear's schedule.
+ * and the size is 0 when no cut of 256 x 256 tiles pays or a smaller tile,
+ * whole, is faster still. A null or smaller workspace (and a size of 0) runs
+ * oga_fp8_linear's schedule.
  */
 int64_t oga_fp8_linear_workspace_bytes(int64_t m, int64_t n, int64_t k);
+
+/*
+ * The schedule of such a call on the persistent kernel (K >= 256, N a multiple
+ * of 128; n: all columns of a grouped call) with workspace_bytes of workspace,
+ * without running it: plan[0] and plan[1] the rows and columns of a tile,
+ * plan[2] the tiles run whole and plan[3] the K-chunks of each other one (1:
+ * none). cus 0 asks the current device, a positive number is a gfx950 of that
+ * many CUs. No counterpart in the reference.
+ */
+int oga_fp8_linear_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_bytes, int64_t cus, int64_t plan[4]);
 
 /*
  * Grouped FP8 linear: `groups` (1..4) linears of n_group output columns each

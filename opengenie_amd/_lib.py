@@ -63,6 +63,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
                                                _i64, _i64, _i64, _f32, _p]),
     "oga_fp8_linear": (_i32, [_p, _i64, _p, _i64, _p, _p, _p, _i32, _p, _i64, _i64, _i64, _i64, _p]),
     "oga_fp8_linear_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "oga_fp8_linear_plan": (_i32, [_i64, _i64, _i64, _i64, _i64, _i64p]),
     "oga_fp8_linear_ws": (_i32, [_p, _i64, _p, _i64, _p, _p, _p, _i32, _p, _i64, _i64, _i64, _i64, _p, _i64, _p]),
     "oga_fp8_linear_dt_ws": (_i32, [_p, _i64, _p, _i64, _p, _p, _p, _i32, _p, _i32, _i64, _i64, _i64, _i64, _p, _i64,
                                     _p]),

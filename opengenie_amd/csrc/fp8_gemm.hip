@@ -1239,17 +1239,30 @@ void set_tiles(GemmArgs& g, int bm, int bn) {
   g.tiles_n = (int)(((int64_t)g.n + bn - 1) / bn);
 }
 
+// The tile of a call and its split, with workspace_bytes to put partials in.
+struct RingPlan {
+  const TileShape* tile;
+  SplitPlan split;
+};
+RingPlan ring_plan(int64_t m, int64_t n, int64_t k, int64_t cus, int64_t workspace_bytes) {
+  SplitPlan p = split_plan(m, n, k, cus);
+  if (workspace_bytes < p.ws_bytes) p.split = 1;
+  const TileShape& t = choose_tile(m, n, k, cus, p);
+  const int64_t nt = ((m + 64 * t.jb - 1) / (64 * t.jb)) * ((n + 64 * t.ib - 1) / (64 * t.ib));
+  if (&t != kTiles || p.split == 1) p = SplitPlan{(int)nt, 1, (int)(k / GKS), (int)nt, 0};
+  return {&t, p};
+}
+
 // The persistent schedule: whole tiles, then (256 x 256 tiles, split,
 // workspace given) the K-chunks of the rest and their sums. g has its shape,
 // operands and groups.
 int launch_ring(GemmArgs& g, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
   const int64_t cus = cu_count();
-  SplitPlan p = split_plan(g.m, g.n, g.k, cus);
-  if (p.split > 1 && (!workspace || workspace_bytes < p.ws_bytes)) p.split = 1;
-  const TileShape& tile = choose_tile(g.m, g.n, g.k, cus, p);
+  const RingPlan plan = ring_plan(g.m, g.n, g.k, cus, workspace ? workspace_bytes : 0);
+  const TileShape& tile = *plan.tile;
+  const SplitPlan& p = plan.split;
   set_tiles(g, 64 * tile.jb, 64 * tile.ib);
   const int64_t nt = (int64_t)g.tiles_m * g.tiles_n;
-  if (&tile != kTiles || p.split == 1) p = SplitPlan{(int)nt, 1, g.k / GKS, (int)nt, 0};
   g.nfull = p.nfull;
   g.split = p.split;
   g.kchunk = p.kchunk;
@@ -1290,7 +1303,21 @@ void set_shape(GemmArgs& g, const void* a, int64_t lda, int64_t ldw, const float
 
 extern "C" int64_t oga_fp8_linear_workspace_bytes(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0 || k % GKS || n % 128 || k < 2 * GKS) return 0;
-  return split_plan(m, n, k, cu_count()).ws_bytes;
+  return ring_plan(m, n, k, cu_count(), INT64_MAX).split.ws_bytes;
+}
+
+extern "C" int oga_fp8_linear_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_bytes, int64_t cus,
+                                   int64_t plan[4]) {
+  if (!plan) return fail("null pointer");
+  if (m <= 0 || n <= 0 || k <= 0 || workspace_bytes < 0 || cus < 0) return fail("bad shape");
+  if (k % GKS || k < 2 * GKS || n % 128 || m > INT32_MAX || n > INT32_MAX || k > INT32_MAX)
+    return unsupported("not a shape of the persistent kernel");
+  const RingPlan p = ring_plan(m, n, k, cus > 0 ? cus : cu_count(), workspace_bytes);
+  plan[0] = 64 * p.tile->jb;
+  plan[1] = 64 * p.tile->ib;
+  plan[2] = p.split.nfull;
+  plan[3] = p.split.split;
+  return OGA_OK;
 }
 
 extern "C" int oga_fp8_linear_dt_ws(const void* a, int64_t lda, const void* w, int64_t ldw, const float* scale_a,

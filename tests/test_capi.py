@@ -104,3 +104,32 @@ def test_attention_plans():
     lib = _lib.load()
     assert lib.oga_attention_plan(0, 1, 1, 1, 1, 256, None) < 0
     assert lib.oga_attention_plan(0, 1, 0, 1, 1, 256, (ctypes.c_int64 * 4)()) < 0
+
+
+def _linear_plan(m, n, k, ws=1 << 62, cus=256):
+    plan = (ctypes.c_int64 * 4)()
+    assert _lib.load().oga_fp8_linear_plan(m, n, k, ws, cus, plan) == 0
+    return tuple(plan)
+
+
+@pytest.mark.skipif(not _lib.available(), reason="library not built")
+def test_fp8_linear_plans():
+    """Schedules on 256 CUs: whole tiles cover the output, K-chunks are cut
+    from 256 x 256 tiles past whole rounds only, and never without a
+    workspace; the tiles of shapes that the kernel's comments name."""
+    for n, k in ((128, 256), (4096, 4096), (4096, 16384), (16384, 4096), (12288, 4096), (4224, 384)):
+        for m in (1, 64, 65, 256, 1152, 1537, 2304, 4100, 4352, 4999, 9216, 14080):
+            for ws in (0, 1 << 62):
+                bm, bn, full, split = _linear_plan(m, n, k, ws)
+                tiles = -(-m // bm) * -(-n // bn)
+                assert split == 1 or (ws and (bm, bn) == (256, 256) and full == tiles // 256 * 256 < tiles)
+                assert split > 1 or full == tiles
+    assert _linear_plan(256, 4096, 4096) == (64, 128, 128, 1)
+    assert _linear_plan(1152, 4096, 4096) == (192, 128, 192, 1)
+    assert _linear_plan(1537, 4096, 4096) == (128, 256, 208, 1)
+    assert _linear_plan(9216, 4096, 4096) == (192, 256, 768, 1)
+    assert _linear_plan(9216, 4096, 16384) == (256, 256, 512, 4)
+    assert _linear_plan(9216, 4096, 16384, 0)[3] == 1
+    lib = _lib.load()
+    assert lib.oga_fp8_linear_plan(1, 128, 128, 0, 256, (ctypes.c_int64 * 4)()) < 0
+    assert lib.oga_fp8_linear_plan(1, 128, 256, 0, 256, None) < 0

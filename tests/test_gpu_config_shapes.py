@@ -20,8 +20,9 @@ Shapes:
   per-head FP8       (1, 9216, 32, 128)
   FP8 quantizer      (9216, 4096) with 0.1 % outliers x50, amax/448 scale
   FP8 linear         9216 x 4096 -> 16384 (nine whole rounds), 16384 -> 4096
-                     and 4096 -> 4096 (split-K tails), grouped Q/K/V 4096 ->
-                     3 x 4096: every output against a full-size checker
+                     (a split-K tail) and 4096 -> 4096 (three whole rounds of
+                     smaller tiles), grouped Q/K/V 4096 -> 3 x 4096: every
+                     output against a full-size checker
                      (decoded e4m3 codes, a float32 device matmul, the
                      reference's two roundings), sampled rows against the
                      oracle (which also pins the checker there), the bias
@@ -29,6 +30,8 @@ Shapes:
 """
 
 from __future__ import annotations
+
+import ctypes
 
 import numpy as np
 import pytest
@@ -312,9 +315,9 @@ def _linear_rows_check(got_rows: np.ndarray, ref_rows: np.ndarray) -> None:
                          ids=["up_4096_to_16384", "down_16384_to_4096", "proj_4096_to_4096"])
 def test_fp8_linear_config_shapes(n, k):
     """The FP8 linear at 9216 tokens on the schedules the benchmark times:
-    4096 -> 16384 is 2304 tiles, nine whole rounds of the persistent kernel;
-    16384 -> 4096 and 4096 -> 4096 are two whole rounds, then the split-K
-    tail (4 and 2 K-chunks) and its reduce. Config 2's data: x ~N(0,1) with
+    4096 -> 16384 is 2304 tiles, nine whole rounds of the persistent kernel on
+    256 CUs; 16384 -> 4096 two whole rounds, then 64 tiles in 4 K-chunks and
+    their reduce; 4096 -> 4096 three whole rounds of 192 x 256. Config 2's data: x ~N(0,1) with
     0.1 % of the entries x50, per-tensor amax/448 scales, W from N(0,0.02),
     bf16 bias ~N(0,0.01). Every output against the full-size device checker
     at the GEMM bar; every 127th row (and the last) against the oracle, and
@@ -326,8 +329,13 @@ def test_fp8_linear_config_shapes(n, k):
 
     m = 9216
     lib = _lib.load()
-    split = int(lib.oga_fp8_linear_workspace_bytes(m, n, k)) > 0
-    assert split == (n == 4096)  # the N = 4096 shapes leave a partial last round
+    plan = (ctypes.c_int64 * 4)()
+    ws_bytes = int(lib.oga_fp8_linear_workspace_bytes(m, n, k))
+    assert lib.oga_fp8_linear_plan(m, n, k, ws_bytes, 0, plan) == 0
+    split = plan[3] > 1
+    assert split == (ws_bytes > 0) == (k == 16384)
+    assert tuple(plan) == {(16384, 4096): (256, 256, 2304, 1), (4096, 16384): (256, 256, 512, 4),
+                           (4096, 4096): (192, 256, 768, 1)}[n, k]
     gg = gen(20260601 + n + k)
     xf = torch.randn((m, k), generator=gg)
     idx = torch.randperm(m * k, generator=gg)[: m * k // 1000]

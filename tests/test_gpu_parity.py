@@ -706,18 +706,32 @@ def test_fp8_linear(m, n, k, bias_dtype):
     assert (bf16_ulp_distance(got, ref) > 1).mean() < 1e-2
 
 
-@pytest.mark.parametrize("m,n,k", [(4352, 4096, 4096), (4352, 4096, 8192), (256, 4096, 4096)])
-def test_fp8_linear_split_k_through_c_abi(m, n, k):
+def _linear_plan(m, n, k, ws_bytes=None):
+    """(rows and columns of a tile, tiles run whole, K-chunks of the others)
+    of an FP8 linear on this device; by default with the workspace it asks for."""
+    import ctypes
+
+    from opengenie_amd import _lib
+
+    lib, plan = _lib.load(), (ctypes.c_int64 * 4)()
+    ws_bytes = lib.oga_fp8_linear_workspace_bytes(m, n, k) if ws_bytes is None else ws_bytes
+    assert lib.oga_fp8_linear_plan(m, n, k, ws_bytes, 0, plan) == 0
+    return tuple(plan)
+
+
+@pytest.mark.parametrize("m,n,k,full,split", [(4352, 4096, 8192, 256, 8), (256, 4096, 16384, 0, 8)])
+def test_fp8_linear_split_k_through_c_abi(m, n, k, full, split):
     """The split-K schedule (workspace given) and the whole-tile schedule
     (no workspace) through the C ABI, both against the oracle. 272 tiles on
-    256 CUs leave 16 for a last round, each cut into K-chunks (4 of 1024 at
-    K = 4096, 8 of 1024 at K = 8192); 256 rows make 16 tiles and no whole
-    round, all of them cut (4 chunks each, the text projections' shape)."""
+    256 CUs leave 16 for a last round, each cut into 8 K-chunks of 1024; 256
+    rows make 16 tiles and no whole round, all of them cut (8 of 2048, the
+    down-projection of a prompt's length). Asserted from the plan."""
     from opengenie_amd import _lib
 
     lib = _lib.load()
     ws_bytes = int(lib.oga_fp8_linear_workspace_bytes(m, n, k))
-    assert ws_bytes > 0  # these shapes leave a partial last round of tiles
+    assert ws_bytes == 16 * split * 256 * 256 * 4
+    assert _linear_plan(m, n, k) == (256, 256, full, split) and _linear_plan(m, n, k, 0)[3] == 1
     x = randn((m, k), 80 + m, std=1.0)
     sa = (x.float().abs().amax() / 448.0).reshape(())
     a = torch.clamp(x.float() / sa, -448, 448).to(torch.float8_e4m3fn)
@@ -743,7 +757,7 @@ def test_fp8_linear_split_k_through_c_abi(m, n, k):
     assert (bf16_ulp_distance(outs[0], outs[1]) > 1).mean() < 1e-3
 
 
-@pytest.mark.parametrize("m,n,k", [(4352, 4096, 4096), (256, 4096, 4096), (9216, 4096, 16384)])
+@pytest.mark.parametrize("m,n,k", [(4352, 4096, 8192), (256, 4096, 16384), (9216, 4096, 16384)])
 def test_fp8_linear_split_k_workspace_reuse(m, n, k):
     """The split-K schedule keeps nothing in its workspace from one call to
     the next: three calls on one workspace and one on a fresh workspace full
@@ -754,7 +768,7 @@ def test_fp8_linear_split_k_workspace_reuse(m, n, k):
 
     lib = _lib.load()
     ws_bytes = int(lib.oga_fp8_linear_workspace_bytes(m, n, k))
-    assert ws_bytes > 0
+    assert ws_bytes > 0 and _linear_plan(m, n, k)[3] > 1
     x = randn((m, k), 380 + m, std=1.0)
     sa = (x.float().abs().amax() / 448.0).reshape(())
     a = torch.clamp(x.float() / sa, -448, 448).to(torch.float8_e4m3fn)
@@ -786,24 +800,31 @@ def test_fp8_linear_split_k_workspace_reuse(m, n, k):
         _linear_full_check(outs[0], _device_fp8_linear(ga, gw, gsa, gsb, gb), "down-projection, split tail")
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (1, 128, 256), (65, 384, 384), (130, 640, 512),  # two, three and four slabs of K: the tiles that run so few
-    (1, 128, 640), (64, 128, 640), (65, 256, 768),   # 64 x 128 tiles: one, exact, one row more
-    (64, 65536, 640),                                # two rounds of them
-    (700, 4096, 640), (1023, 4096, 1024),            # 128 x 128
-    (1100, 4096, 1024), (1152, 16384, 512),          # 192 x 128, one round and several
-    (1537, 4096, 896),                               # 128 x 256
-    (2305, 4096, 640), (2400, 4224, 384),            # 192 x 256, and a last tile half past N
-    (6144, 4096, 256),                               # two whole rounds of them
-    (64, 4096, 16384)])                              # K-chunks of 256 x 256
+@pytest.mark.parametrize("m,n,k,plan", [  # (plans on 256 CUs)
+    # two, three and four slabs of K: the tiles that run so few
+    (1, 128, 256, (192, 256, 1, 1)), (65, 384, 384, (192, 128, 3, 1)), (130, 640, 512, (128, 128, 10, 1)),
+    # 64 x 128: one, exact, one row more, two rounds of them
+    (1, 128, 640, (64, 128, 1, 1)), (64, 128, 640, (64, 128, 1, 1)), (65, 256, 768, (64, 128, 4, 1)),
+    (64, 65536, 640, (64, 128, 512, 1)),
+    (700, 4096, 640, (128, 128, 192, 1)), (1023, 4096, 1024, (128, 128, 256, 1)),
+    (1100, 4096, 1024, (192, 128, 192, 1)), (1152, 16384, 512, (192, 128, 768, 1)),
+    # 128 x 256, one round and three (staged in an A buffer of the running ring)
+    (1537, 4096, 896, (128, 256, 208, 1)), (1951, 12288, 4096, (128, 256, 768, 1)),
+    # 192 x 256, a last tile half past N, two rounds
+    (2305, 4096, 640, (192, 256, 208, 1)), (2400, 4224, 384, (192, 256, 221, 1)),
+    (6144, 4096, 256, (192, 256, 512, 1)),
+    # 256 x 256: one round, a round and K-chunks, K-chunks alone
+    (1024, 16384, 1024, (256, 256, 256, 1)), (4352, 4096, 8192, (256, 256, 256, 8)),
+    (64, 4096, 16384, (256, 256, 0, 8))])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_fp8_linear_tiles(m, n, k, dtype):
+def test_fp8_linear_tiles(m, n, k, plan, dtype):
     """The tiles of the persistent kernel at their edges (ragged rows and
     columns, the fewest slabs of K each runs, one and several rounds of the
     CUs) through fp8_scaled_mm, the biased output against the oracle and, bit
     for bit, against R(unbiased + bias)."""
     from opengenie_amd.ltx_ops import fp8_scaled_mm
 
+    assert _linear_plan(m, n, k) == plan
     x = randn((m, k), 390 + m, std=1.0)
     sa = (x.float().abs().amax() / 448.0).reshape(())
     a = torch.clamp(x.float() / sa, -448, 448).to(torch.float8_e4m3fn)
@@ -831,8 +852,8 @@ def _bias_epilogue_ref(out_nobias: np.ndarray, bias: torch.Tensor, r=bf16_round)
 
 
 @pytest.mark.parametrize("m,n,k", [(300, 520, 384), (512, 768, 1024), (1, 16, 128),
-                                   (4352, 4096, 4096),  # whole-tile rounds + split-K last round
-                                   (256, 4096, 4096),   # split-K only
+                                   (4352, 4096, 4096),  # rounds of whole 192 x 128 tiles
+                                   (256, 4096, 16384),  # split-K only
                                    (600, 16384, 384)])
 @pytest.mark.parametrize("bias_dtype", [None, torch.bfloat16, torch.float32, torch.float16])
 def test_fp8_linear_fp16_output(m, n, k, bias_dtype):
@@ -872,8 +893,8 @@ def test_fp8_linear_fp16_output(m, n, k, bias_dtype):
 
 @pytest.mark.parametrize("m,n,k,use_ws", [
     (4352, 4096, 4096, False),  # persistent whole-tile schedule
-    (4352, 4096, 4096, True),   # + split-K last round
-    (256, 4096, 4096, True),    # split-K only
+    (4352, 4096, 8192, True),   # + split-K last round
+    (256, 4096, 16384, True),   # split-K only
     (300, 520, 384, False),     # one workgroup per tile (N not a multiple of 128)
 ])
 def test_fp8_linear_fp16_bias_epilogue_is_exact(m, n, k, use_ws):
@@ -890,7 +911,7 @@ def test_fp8_linear_fp16_bias_epilogue_is_exact(m, n, k, use_ws):
     ga, gw, gsa, gsb, gb = g(a), g(w), g(sa).float(), g(sb).float(), g(bias)
     ws_bytes = int(lib.oga_fp8_linear_workspace_bytes(m, n, k)) if use_ws else 0
     if use_ws:
-        assert ws_bytes > 0
+        assert ws_bytes > 0 and _linear_plan(m, n, k)[3] > 1
     ws = torch.empty((max(ws_bytes, 4) // 4,), device="cuda", dtype=torch.float32)
     stream = torch.cuda.current_stream().cuda_stream
     outs = []
@@ -963,8 +984,8 @@ def test_fp8_linear_forward_fp16_module():
 
 @pytest.mark.parametrize("m,n,k,bias_dtype,use_ws", [
     (4352, 4096, 4096, torch.bfloat16, False),  # persistent whole-tile schedule
-    (4352, 4096, 4096, torch.bfloat16, True),   # + split-K last round (16 tiles x 4 K-chunks)
-    (256, 4096, 4096, torch.bfloat16, True),    # split-K only (16 tiles x 4 K-chunks, no whole round)
+    (4352, 4096, 8192, torch.bfloat16, True),   # + split-K last round (16 tiles x 8 K-chunks)
+    (256, 4096, 16384, torch.bfloat16, True),   # split-K only (16 tiles x 8 K-chunks, no whole round)
     (300, 520, 384, torch.float32, False),      # one-workgroup-per-tile kernel (N not a multiple of 128)
     (300, 520, 384, torch.bfloat16, False),
 ])
@@ -983,7 +1004,7 @@ def test_fp8_linear_bias_epilogue_is_exact(m, n, k, bias_dtype, use_ws):
     ga, gw, gsa, gsb, gb = g(a), g(w), g(sa).float(), g(sb).float(), g(bias)
     ws_bytes = int(lib.oga_fp8_linear_workspace_bytes(m, n, k)) if use_ws else 0
     if use_ws:
-        assert ws_bytes > 0
+        assert ws_bytes > 0 and _linear_plan(m, n, k)[3] > 1
     ws = torch.empty((max(ws_bytes, 4) // 4,), device="cuda", dtype=torch.float32)
     stream = torch.cuda.current_stream().cuda_stream
     outs = []
@@ -996,18 +1017,25 @@ def test_fp8_linear_bias_epilogue_is_exact(m, n, k, bias_dtype, use_ws):
     assert_same_bits(outs[1], _bias_epilogue_ref(outs[0], bias), "bias epilogue")
 
 
-def test_fp8_grouped_linear_bias_epilogue_is_exact():
+@pytest.mark.parametrize("m,plan", [(1536, (192, 128, 768, 1)),
+                                    (1951, (128, 256, 768, 1)),   # three rounds of swizzled staging
+                                    (4100, (256, 256, 768, 4))])  # the last four rows' 48 tiles in K-chunks
+def test_fp8_grouped_linear_bias_epilogue_is_exact(m, plan):
     """The grouped kernel's per-linear bias: with and without the biases,
-    out_bias == R(out_nobias + R(bias_i)) for every linear and element."""
+    out_bias == R(out_nobias + R(bias_i)) for every linear and element; and
+    each linear's rows, sampled and the last ones, against the oracle (its
+    own weight scale, bias and output in whole and in K-split tiles)."""
     import ctypes
 
     from opengenie_amd import _lib
 
     lib = _lib.load()
-    m, n, k, groups = 1536, 4096, 4096, 3
+    n, k, groups = 4096, 4096, 3
+    assert _linear_plan(m, groups * n, k) == plan
     x = randn((m, k), 190, std=1.0)
     sa = (x.float().abs().amax() / 448.0).reshape(())
-    a = g(torch.clamp(x.float() / sa, -448, 448).to(torch.float8_e4m3fn))
+    codes = torch.clamp(x.float() / sa, -448, 448).to(torch.float8_e4m3fn)
+    a = g(codes)
     gsa = g(sa).float()
     ws_ = [_fp8_weights(n, k, 191 + i) for i in range(groups)]
     w = [g(t[0]) for t in ws_]
@@ -1029,6 +1057,11 @@ def test_fp8_grouped_linear_bias_epilogue_is_exact():
         res.append([out_np(o) for o in outs])
     for i in range(groups):
         assert_same_bits(res[1][i], _bias_epilogue_ref(res[0][i], biases[i]), f"grouped bias epilogue {i}")
+    rows = np.unique(np.concatenate([np.arange(0, m, 61), np.arange(m - 8, m)]))
+    for i in range(groups):
+        ref = O.fp8_linear(codes.view(torch.uint8).numpy()[rows], ws_[i][0].view(torch.uint8).numpy(), float(sa),
+                           float(ws_[i][1]), to_T(biases[i].cpu()))
+        _close_to(res[1][i][rows], ref, f"grouped linear {i}")
 
 
 class _FP8Lin(torch.nn.Module):
@@ -1048,7 +1081,7 @@ class _FP8Lin(torch.nn.Module):
 def test_fp8_qkv_grouped_mm(tokens, names):
     """fp8_qkv_from_grouped_mm / fp8_qk_from_grouped_mm: one launch, each
     linear with its own weight scale and bias, against the oracle per linear
-    (1536 tokens: more tiles than CUs, split-K tail)."""
+    (1536 tokens: more tiles than CUs)."""
     from opengenie_amd import ltx_ops as L
 
     attn = torch.nn.Module()
