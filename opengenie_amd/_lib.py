@@ -1,6 +1,7 @@
 """Binding of libopengenie_amd.so (the C ABI in include/opengenie_amd.h): load()
 gives it through ctypes; call() and function() go through the compiled module
-_native, whose calls cost the wrappers less (pycall.cpp).
+_native, whose calls cost the wrappers less (pycall.cpp), or through ctypes
+where this interpreter has no such module.
 
 The library is loaded on first use. If it is missing the call raises: a GPU
 tensor never silently takes another path because the extension is absent.
@@ -25,7 +26,23 @@ _i64 = ctypes.c_int64
 _i32 = ctypes.c_int
 _f32 = ctypes.c_float
 _p = ctypes.c_void_p
-_i64p = ctypes.POINTER(ctypes.c_int64)
+
+
+# ctypes makes an array type anew on every `c_int64 * n`; these are kept.
+_I64_ARRAYS = tuple(ctypes.c_int64 * n for n in range(6))
+
+
+class _i64p:
+    """int64_t array argument: a tuple of ints, as _native takes it, or what
+    POINTER(c_int64) takes."""
+
+    _pointer = ctypes.POINTER(ctypes.c_int64)
+
+    @classmethod
+    def from_param(cls, value):
+        return strides(value) if isinstance(value, tuple) else cls._pointer.from_param(value)
+
+
 
 # name -> (restype, argtypes); must match include/opengenie_amd.h
 SIGNATURES: dict[str, tuple[object, list[object]]] = {
@@ -121,10 +138,6 @@ def available() -> bool:
     return os.path.exists(LIB_PATH)
 
 
-# ctypes makes an array type anew on every `c_int64 * n`; these are kept.
-_I64_ARRAYS = tuple(ctypes.c_int64 * n for n in range(6))
-
-
 def strides(values) -> ctypes.Array:
     return _I64_ARRAYS[len(values)](*values)
 
@@ -138,8 +151,8 @@ def function(name: str):
         lib = load()
         try:
             from . import _native  # built with the library, linked to the same file
-        except ImportError as e:
-            raise LibraryMissing(f"the _native module is not built; run `python -m opengenie_amd.build` ({e})") from e
+        except ImportError:  # another interpreter, or no Python.h when the library was built
+            _native = None
         fn = _fns[name] = getattr(_native, name, None) or getattr(lib, name)
     return fn
 

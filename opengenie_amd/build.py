@@ -5,7 +5,9 @@ Usage: python -m opengenie_amd.build [--jobs N]
 
 Every .hip source is compiled to an object in parallel, then linked into one
 shared library next to this file; pycall.cpp (host code) becomes the module
-_native beside it, linked to the library. Flags of the device sources:
+_native of this interpreter beside it, linked to the library (without the
+interpreter's headers there is none, and the wrappers call through ctypes).
+Flags of the device sources:
   --offload-arch=gfx950         CDNA4 (MI355X) only
   -ffp-contract=off             no silent a*b+c fusion (bit-exact rounding)
   -target-feature -packed-fp32-ops
@@ -15,6 +17,7 @@ _native beside it, linked to the library. Flags of the device sources:
 from __future__ import annotations
 
 import argparse
+import glob
 import os
 import shutil
 import subprocess
@@ -74,17 +77,30 @@ def build(jobs: int | None = None, verbose: bool = False) -> str:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
+    if not _build_native() and verbose:
+        print("no Python.h: _native not built, calls go through ctypes", file=sys.stderr)
+    if verbose:
+        print(f"built {LIB_PATH} from {len(srcs)} sources", file=sys.stderr)
+    return LIB_PATH
+
+
+def _build_native() -> bool:
+    """Builds _native for this interpreter; those of an earlier library go, as
+    their entry points may have other arguments. False without Python.h."""
+    for old in glob.glob(os.path.join(HERE, "_native.*")):
+        os.remove(old)
+    include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        return False
     tmp = NATIVE_PATH + ".tmp"
     cmd = [hipcc(), "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wl,--as-needed",
-           "-I" + sysconfig.get_paths()["include"], os.path.join(CSRC, "pycall.cpp"), "-o", tmp,
+           "-I" + include, os.path.join(CSRC, "pycall.cpp"), "-o", tmp,
            "-L" + HERE, "-lopengenie_amd", "-Wl,-rpath,$ORIGIN"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"_native failed:\n{' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, NATIVE_PATH)
-    if verbose:
-        print(f"built {LIB_PATH} from {len(srcs)} sources", file=sys.stderr)
-    return LIB_PATH
+    return True
 
 
 def main() -> None:

@@ -7,6 +7,7 @@ from __future__ import annotations
 import ctypes
 import os
 import re
+import sys
 
 import pytest
 
@@ -75,6 +76,35 @@ def test_native_module_binds_the_same_library():
         _native.oga_adazero_from_ada(4096, 4096, 1, 1, 4096, 4096, 0, 1, 1, 4096, 0, (1,) * 9, 0, 1, 1e-6, None)
     with pytest.raises(_lib.KernelError):
         _lib.call("oga_bias_add_bf16", None, None, 0, None, 1, 1, None)
+
+
+@pytest.mark.skipif(not _lib.available(), reason="library not built")
+def test_wrappers_call_through_ctypes_without_the_native_module(monkeypatch):
+    """An interpreter the compiled module was not built for calls the same
+    library through ctypes, with the arguments the wrappers pass to either."""
+    monkeypatch.setitem(sys.modules, "opengenie_amd._native", None)  # its import fails
+    monkeypatch.delattr("opengenie_amd._native", raising=False)
+    monkeypatch.setattr(_lib, "_fns", {})
+    assert _lib.function("oga_adazero_from_ada") is _lib.load().oga_adazero_from_ada
+    for st in ((1, 1, 1, 1), _lib.strides((1, 1, 1, 1))):
+        with pytest.raises(_lib.KernelError, match="4096"):  # channels
+            _lib.call("oga_adazero_from_ada", 4096, 4096, 1, 1, 100, 4096, 0, 1, 1, 4096, 0, st, 0, 1, 1e-6, None)
+    with pytest.raises(_lib.KernelError, match="null"):
+        _lib.call("oga_attention_ws", None, (1, 1, 1), None, (1, 1, 1), None, (1, 1, 1), None, (1, 1, 1), 1, 1, 1, 1,
+                  128, 1.0, None, 0, None)
+    assert _lib.function("oga_attention_workspace_bytes")(0, 1, 1, 1, 128) == 0
+
+
+def test_the_library_builds_without_python_headers(monkeypatch, tmp_path):
+    """Without Python.h there is no compiled module, an older one goes, and
+    building says so instead of failing."""
+    from opengenie_amd import build
+
+    old = tmp_path / "_native.cpython-39-x86_64-linux-gnu.so"
+    old.write_bytes(b"")
+    monkeypatch.setattr(build, "HERE", str(tmp_path))
+    monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    assert build._build_native() is False and not old.exists()
 
 
 def _attention_plan(fp8, batch, nq, nk, heads, cus=256):
