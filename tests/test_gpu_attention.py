@@ -524,7 +524,6 @@ def test_attention_config_shape():
     query rows of heads 0 (first round) and 31 (every block in the key-split
     round), and every 31st row of heads 13 and 30, against float64 attention
     at the bf16 bar above."""
-    from opengenie_amd import _lib
     from opengenie_amd.attention import flash_attn_func
 
     n, h = 9216, 32

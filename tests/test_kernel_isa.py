@@ -129,12 +129,15 @@ def test_attention_barriers_wait_for_lds_dma():
 @pytest.mark.skipif(not os.path.exists("/opt/rocm/bin/hipcc") and not os.environ.get("HIPCC"),
                     reason="hipcc not present")
 def test_fp8_attention_barriers_wait_for_lds_dma():
-    """The FP8 kernel sends two DMA instructions per wave and step (the K
-    tile and the V^T tile), so the wait may leave the next step's two in flight."""
-    body = _kernel_body(_device_asm(os.path.join(CSRC, "attention.hip")), "k_attention_fp8")
-    assert sum(1 for ins in body if ins == "s_barrier") >= 2
-    assert any("load_lds" in ins for ins in body)
-    assert barrier_violations(body, max_vmcnt=2) == []
+    """Both forms of the FP8 kernel: a wave of the 12-wave one sends two DMA
+    instructions per step (one of the K tile, one of the V^T tile), of the
+    4-wave one four, so the wait may leave the next step's two or four in flight."""
+    asm = _device_asm(os.path.join(CSRC, "attention.hip"))
+    for mangled, dma in (("k_attention_fp8ILi12EE", 2), ("k_attention_fp8ILi4EE", 4)):
+        body = _kernel_body(asm, mangled)
+        assert sum(1 for ins in body if ins == "s_barrier") >= 2, mangled
+        assert sum("load_lds" in ins for ins in body) >= 2 * dma, mangled
+        assert barrier_violations(body, max_vmcnt=dma) == [], mangled
 
 
 # ----------------------------------------------------------------- LDS reads
@@ -233,3 +236,83 @@ def test_no_register_of_an_outstanding_lds_read_is_named(src):
         assert lds_read_hazards(body) == [], (src, lines[start])
         checked += 1
     assert checked >= 1
+
+
+# ------------------------------------------------- loads waited for by count
+def load_hazards(body: list[str], after: tuple[int, int] = (-1, 0)) -> list[int]:
+    """Indexes of instructions that name a VGPR which a global load still in
+    flight will write: on some path from the load, before an s_waitcnt
+    vmcnt(n) with at least n vector memory instructions issued since the load
+    (they retire in order). For the fewest such instructions on any path to
+    each instruction; a load through inline assembly is the kernel's to wait
+    for. after = (n, barriers): no path reaches an s_waitcnt vmcnt(n) with
+    fewer barriers since the load (the trips a loop is known to make)."""
+    labels = {ins[:-1]: i for i, ins in enumerate(body) if ins.endswith(":")}
+    bad = set()
+    for start, ins in enumerate(body):
+        if not ins.startswith("global_load_dword"):
+            continue
+        regs = _vregs(ins.partition(" ")[2].split(",")[0])
+        fewest: dict[tuple[int, int], int] = {}
+        todo = [(start + 1, 0, 0)]
+        while todo:
+            i, issued, barriers = todo.pop()
+            if i >= len(body) or fewest.get((i, barriers), issued + 1) <= issued:
+                continue
+            fewest[i, barriers] = issued
+            op, _, args = body[i].partition(" ")
+            if op == "s_endpgm":
+                continue
+            wait = re.search(r"\bvmcnt\((\d+)\)", args) if op == "s_waitcnt" else None
+            if wait and (int(wait[1]) <= issued or (int(wait[1]) == after[0] and barriers < after[1])):
+                continue
+            if op == "s_barrier":
+                barriers = min(barriers + 1, after[1])
+            if not op.endswith(":") and not op.startswith((".", "s_")) and _vregs(args) & regs:
+                bad.add(i)
+                continue
+            if op.startswith(("global_", "buffer_", "flat_", "scratch_")):
+                issued += 1
+            if op.startswith(("s_branch", "s_cbranch")):
+                todo.append((labels[args.strip()], issued, barriers))
+            if op != "s_branch":
+                todo.append((i + 1, issued, barriers))
+    return sorted(bad)
+
+
+def test_load_hazard_check_follows_every_path():
+    load, dma = "global_load_dwordx4 v[4:7], v[2:3], off", "buffer_load_dwordx4 v9, s[0:3], 0 offen lds"
+    use = "v_mov_b32_e32 v0, v5"
+    assert load_hazards([load, use]) == [1]
+    assert load_hazards([load, "s_waitcnt vmcnt(0)", use]) == []
+    assert load_hazards([load, dma, "s_waitcnt vmcnt(1)", use]) == []
+    assert load_hazards([load, dma, "s_waitcnt vmcnt(2)", use]) == [3]
+    # the wait is in a loop that the load's path may leave first
+    body = [load, ".L1:", dma, "s_cbranch_scc1 .L2", "s_waitcnt vmcnt(1)", "s_branch .L1", ".L2:", use]
+    assert load_hazards(body) == [7]
+    # text order is not the order of execution: the use stands before the load
+    body = ["s_branch .L2", ".L1:", use, "s_endpgm", ".L2:", load, dma, "s_waitcnt vmcnt(1)", "s_branch .L1"]
+    assert load_hazards(body) == []
+    body[7] = "s_waitcnt lgkmcnt(0)"
+    assert load_hazards(body) == [2]
+    # a loop of one DMA a trip: its end's wait covers the load after three trips
+    body = [load, ".L1:", dma, "s_barrier", "s_cbranch_scc1 .L1", "s_waitcnt vmcnt(3)", use]
+    assert load_hazards(body) == [6] and load_hazards(body, (3, 2)) == [6] and load_hazards(body, (3, 3)) == []
+
+
+@pytest.mark.skipif(not os.path.exists("/opt/rocm/bin/hipcc") and not os.environ.get("HIPCC"),
+                    reason="hipcc not present")
+def test_bias_loads_of_every_gemm_tile_are_waited_for():
+    """The persistent GEMM loads a tile's bias through inline assembly and
+    names no wait for it: the counted waits of its first odd step, or with
+    more than two slabs sent ahead the one before the epilogue (two slabs of
+    2 ib + 2 jb DMA instructions, after at least as many slabs, each with a
+    barrier, as are sent ahead), must cover it in every instance."""
+    asm = _device_asm(os.path.join(CSRC, "fp8_gemm.hip"))
+    for ib, jb in ((4, 4), (4, 3), (4, 2), (2, 3), (2, 2), (2, 1)):
+        for f16 in (0, 1):
+            body = _kernel_body(asm, f"k_fp8_gemm_ringILi{ib}ELi{jb}ELb0ELb{f16}EE")
+            assert sum(ins.startswith("global_load_dwordx4") for ins in body) >= ib // 2
+            ahead = 6 - jb if ib == 2 else 3 if jb == 2 else 2
+            after = (2 * (2 * ib + 2 * jb), ahead) if ahead > 2 else (-1, 0)
+            assert load_hazards(body, after) == [], (ib, jb, f16)
