@@ -1188,8 +1188,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(3, 3))) 
   auto step = [&](auto par_c, int64_t st) {
     constexpr int PAR = decltype(par_c)::value;
     // This wave's DMA of step st has landed (the last two instructions of
-    // step st + 1's, sent a step ago, may still be in flight), then every
-    // wave's.
+    // step st + 1's, sent a step ago, may still be in flight: all of them in
+    // the wide form; the narrow one's four make this wait cover the first two,
+    // the K tile's, as well, more than step st needs), then every wave's.
     asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
     asm volatile("s_barrier" ::: "memory");
     constexpr int NP = (PAR + kF8Bufs - 1) % kF8Bufs;
@@ -1445,13 +1446,14 @@ int split_candidate(int64_t rem, int64_t nk, int64_t slots) {
 }
 // Time of `units` units of `steps` key steps each, in us: rounds of the
 // resident workgroups, the last one at the step time of as many workgroups
-// per CU as it still needs. A step of one 8-wave bf16 workgroup takes ~1.6 us,
-// of one 12-wave FP8 workgroup ~1.65; of one, two or three 4-wave FP8
-// workgroups on a CU ~0.75, 1.2 and 1.72 us; a unit's Q loads, first tiles
-// and O stores ~4 us.
+// per CU as it still needs. A step of one 8-wave bf16 workgroup takes ~1.85 us
+// (1228 us at 9216 tokens x 32 heads, 648 steps and five units' ends; 50 at
+// 1537, 25 steps), of one 12-wave FP8 workgroup ~1.65; of one, two or three
+// 4-wave FP8 workgroups on a CU ~0.75, 1.2 and 1.72 us; a unit's Q loads, first
+// tiles and O stores ~4 us.
 double units_us(AttnKernel kern, int64_t units, double steps, int64_t slots) {
   static constexpr double kNarrowStep[3] = {0.75, 1.2, 1.72};
-  const double full = kern == kFp8Narrow ? kNarrowStep[2] : kern == kFp8Wide ? 1.65 : 1.6;
+  const double full = kern == kFp8Narrow ? kNarrowStep[2] : kern == kFp8Wide ? 1.65 : 1.85;
   double t = (double)(units / slots) * (steps * full + 4.0);
   const int64_t rest = units % slots;
   if (rest) {

@@ -516,18 +516,20 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
 // tiles v, v + G, v + 2G, ... (G = grid size; with the XCD remap every tile
 // of a workgroup lies in its XCD's range, and at any moment the XCD's
 // workgroups work on consecutive tiles of that range) and keeps the slab
-// ring running across tile boundaries: the DMA of a tile's last two slabs
-// fetches slabs 0 and 1 of its next tile, so when the epilogue ends the next
-// tile's first operands are in LDS and its first fragments in VGPRs. The
-// epilogue stages each wave's output, 32 rows at a time, in its own quarter
-// of the A buffer of the tile's last slab: no wave reads that buffer any
-// more (the last odd step's barrier), no DMA targets it until the next
-// tile's first even step, and the first DMA into that quarter is the same
-// wave's own, issued after its staging reads completed. The stores are not
-// waited for here; the next tile's first odd step waits for them with the
-// DMA sent before them.
+// ring running across tile boundaries: the DMA of a tile's last kAhead slabs
+// (two to five, by the tile: RingTile) fetches the first slabs of its next
+// tile, so when the epilogue ends the next tile's first operands are in LDS
+// and its first fragments in VGPRs. The epilogue stages each wave's output, 32
+// rows at a time: after the ring where LDS has room (192 x 256 and 64 x 128),
+// else in the wave's own quarter of the A buffer of the tile's last slab. No
+// wave reads that buffer any more (the last odd step's barrier), no DMA
+// targets it until the next tile's first even step, and the first DMA into
+// that quarter is the same wave's own, issued after its staging reads
+// completed. The stores are not waited for here; a counted wait of the next
+// tile covers them, the first odd step's with two slabs ahead.
 constexpr int kStagePitch = 136;  // bytes per staged row of 64 bf16 columns
-// Staged row r, 16-byte chunk c (of 8) sits at byte r * kStagePitch + 16c.
+// Staged row r, 16-byte chunk c (of 8) sits at byte r * kStagePitch + 16c, or
+// in a quarter of 4 KiB (128 x 256 and 128 x 128) at 128r + 16 (c ^ (r/2 % 8)).
 // Writes: lane (fr, fh) stores 8 bytes of row fr at chunk c, half fh; each
 // 32-lane half of a ds_write_b64 must touch 64 distinct banks. Reads: lane l
 // loads row 4u + l/16 + 16*((l/8)%2), chunk l%8; each 16-lane group of a
@@ -559,6 +561,22 @@ constexpr bool stage_reads_conflict_free() {
     }
   return true;
 }
+// Of the 4 KiB quarters: lane l reads row 8u + l/8, chunk l%8. (The writes are
+// two-way conflicted: rows r and r + 16 keep a chunk in the same banks.)
+constexpr bool packed_reads_conflict_free() {
+  for (int u = 0; u < 4; ++u)
+    for (int grp = 0; grp < 4; ++grp) {
+      unsigned long long banks = 0;
+      for (int l = 16 * grp; l < 16 * grp + 16; ++l) {
+        const int row = 8 * u + (l >> 3);
+        const int b = ((row * 128 + (((l & 7) ^ ((row >> 1) & 7)) << 4)) >> 2) & 63;
+        if ((banks >> b) & 15ull) return false;
+        banks |= 15ull << b;  // b is a multiple of 4: no wrap
+      }
+    }
+  return true;
+}
+static_assert(packed_reads_conflict_free(), "packed staging reads would conflict");
 static_assert(stage_writes_conflict_free(), "staging writes would conflict");
 static_assert(stage_reads_conflict_free(), "staging reads would conflict");
 // Word 3 of a buffer resource on gfx9: 32-bit data format, no swizzle.
@@ -814,7 +832,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   };
 
   // Staging: a pass holds 32 rows x 64 columns of the wave's block (block
-  // row j, column half h) inside the wave's 8 KiB quarter. Lane (fr, fh)
+  // row j, column half h) inside the wave's staging. Lane (fr, fh)
   // writes at sw + 64*(i - 2h) + 16q; lane l reads its row (srow, plus 4u)
   // at sr + 4u * kStagePitch.
   // Swizzled (packed) rows keep chunk c of row r at c ^ ((r / 2) % 8), and a
@@ -837,7 +855,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   int s = 0;
   int m0, n0, kb, kn, sp;
   unit(v, m0, n0, kb, kn, sp);
-  // W of the group holding columns n0 .. n0 + 255, from its first row.
+  // W of the group holding columns n0 .. n0 + kBN - 1, from its first row.
   auto wrsrc = [&](int n0) {
     const int gi = n0 / g.group_n, r0 = n0 - gi * g.group_n;
     return rsrc(pick(g.wg, gi), r0, g.group_n, T::kBN, g.ldw);
@@ -1226,9 +1244,10 @@ const TileShape& choose_tile(int64_t m, int64_t n, int64_t k, int64_t cus, const
       us += (double)split.kchunk * slab(rest * split.split) + kSplitUs + kSplitChunkUs * (double)(rest * split.split);
     else if (rest)
       us += (double)nslab * slab(rest) + t.round;
-    // (5 % less than the 256 x 256 tile's: over long kernels the clock follows
-    // the MFMAs' power, and three rounds of 192 x 256 at 9216 x 16384 -> 4096,
-    // modelled 4 % shorter, measured 0.7 % longer.)
+    // (5 % less than the 256 x 256 tile's: the model's error, 3 to 8 % rms per
+    // tile, can make a smaller tile look shorter that is not, as at 9216 x
+    // 16384 -> 4096, whose three rounds of 192 x 256 are modelled 4 % shorter
+    // and measured 0.7 % longer.)
     if (!best || us < best_us * (best == kTiles ? 0.95 : 1.0)) { best = &t; best_us = us; }
   }
   return *best;  // (K >= 256: the two-slab tiles always qualify)
