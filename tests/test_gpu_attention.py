@@ -462,6 +462,38 @@ def test_attention_error_is_that_of_key_parts(n):
         assert err <= 1.01 * want, (n, head, err, want)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("falling", [True, False])
+def test_attention_restarts_with_falling_and_rising_scores(fp8, falling):
+    """Whole blocks that begin a new running max per key part (1537 tokens x 32
+    heads), with scores that fall or rise by tens of octaves from the first key
+    to the last, further per part than a restart may lower the max: float64
+    attention at the bars of the two kernels."""
+    from opengenie_amd.attention import flash_attn_func
+
+    n, h, heads = 1537, 32, [0, 31]
+    assert _plan(fp8, 1, n, n, h)[2:] == (_plan(fp8, 1, n, n, h)[1], 1)
+    q, k, v = (randn((1, n, h, 128), 980 + i).to(DEV) for i in range(3))
+    ramp = torch.linspace(3.0, -3.0, n, device=DEV)[None, :, None, None]  # score q.k/sqrt(128): about +-34
+    q = (q.float() * 0.25 + 1.0).to(torch.bfloat16)
+    k = (k.float() * 0.25 + (ramp if falling else -ramp)).to(torch.bfloat16)
+    if fp8:
+        q, k, v = (t.to(torch.float8_e4m3fn) for t in (q, k, v))
+        one = torch.ones((1, h), device=DEV)
+        out = flash_attn_func(q, k, v, q_descale=one, k_descale=one, v_descale=one)
+        _ran("flash_attn_func_fp8")
+    else:
+        out = flash_attn_func(q, k, v)
+        _ran("flash_attn_func")
+    qe, ke, ve = (t[:, :, heads].double().cpu().numpy() for t in (q, k, v))
+    ref = O.attention(*[np.ascontiguousarray(x.transpose(0, 2, 1, 3)) for x in (qe, ke, ve)]).transpose(0, 2, 1, 3)
+    got = out[:, :, heads].float().cpu().numpy()
+    if fp8:
+        _check_fp8(got, ref, _fp8_rounding_bound(qe, ke, ve), f"fp8 restarts, falling {falling}")
+    else:
+        _check(torch.from_numpy(got), ref, f"bf16 restarts, falling {falling}")
+
+
 def test_fp8_attention_strided_views():
     """q, k, v as strided [B, N, H, D] views of one packed e4m3 buffer."""
     from opengenie_amd.attention import flash_attn_func
