@@ -33,8 +33,10 @@
 // Two kernels share this loop: k_fp8_gemm_ring (K >= 256, N % 128 == 0, bf16
 // or no bias) is persistent, one workgroup per CU looping over tiles with
 // the slab ring running on across tile boundaries, and is built for six
-// tiles from 256 x 256 down to 64 x 128 (choose_tile); k_fp8_gemm (every
-// other supported shape) runs one workgroup per 256 x 256 tile.
+// tiles from 256 x 256 down to 64 x 128 (choose_tile; the smaller ones' slabs
+// are sent further ahead and lie closer in LDS than said here for 256 x 256:
+// RingTile); k_fp8_gemm (every other supported shape) runs one workgroup per
+// 256 x 256 tile.
 //
 // LDS layout of an operand slab (256 rows x 128 bytes): two rows share one
 // 256-byte line of the 64 LDS banks; row r's 16-byte chunk c (c = 0..7)
